@@ -1,0 +1,112 @@
+"""The one-pass form of a dilation (the default up to R = 255) against the two
+sweeps (VO_PASS1=zsweep), bit for bit, and against the oracle: tiles of 8 x 8
+columns cut by the grid, radii at the edges of its variants, lists past their
+LDS entries and past their first room, columns of more segments than its
+summaries count, empty and touching columns."""
+
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+from voroffset_amd import _native, synth
+from voroffset_amd.volume import CompressedVolume
+
+from .helpers import compare_csr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def contexts():
+    one = _native.Context(0)
+    old = os.environ.get("VO_PASS1")
+    os.environ["VO_PASS1"] = "zsweep"
+    try:
+        two = _native.Context(0)
+    finally:
+        if old is None:
+            del os.environ["VO_PASS1"]
+        else:
+            os.environ["VO_PASS1"] = old
+    yield one, two
+    one.close()
+    two.close()
+
+
+def both(contexts, vol, op, prec, r):
+    zlo, zhi = vol.z_range()
+    res = [c.morph_host(op, prec, r, vol.nx, vol.ny, vol.off, vol.z, zlo, zhi)[:2] for c in contexts]
+    assert np.array_equal(res[0][0], res[1][0])
+    assert np.array_equal(res[0][1], res[1][1])
+    return res[0]
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("nx,ny", [(1, 1), (7, 9), (8, 8), (65, 3), (3, 70), (129, 41)])
+@pytest.mark.parametrize("r", [0.0, 0.9, 3.0, 5.0, 7.9, 8.0, 12.3, 31.5, 32.0, 64.0])
+def test_grids_and_radii(contexts, prec, nx, ny, r):
+    vol = synth.poisson_columns(nx, ny, lam=4, zmax=500, seed=nx + 7 * ny, z_margin=int(r) + 3)
+    off, z = both(contexts, vol, "dilation", prec, r)
+    if prec == "fp64" and nx * ny <= 300:
+        bad, err = compare_csr(off, z, *oracle.morph(vol, "dilation", r))
+        assert len(bad) == 0 and err <= 1e-9
+
+
+@pytest.mark.parametrize("op", ["erosion", "closing", "opening"])
+@pytest.mark.parametrize("r", [2.5, 9.0])
+def test_solids(contexts, op, r):
+    vol = synth.ball_union(9, 60, seed=int(r), rmin=5.0, rmax=14.0, pad=14)
+    for prec in ("fp32", "fp64"):
+        both(contexts, vol, op, prec, r)
+
+
+@pytest.mark.parametrize("r", [100.0, 255.0])
+def test_large_radii(contexts, r):
+    vol = synth.poisson_columns(300, 20, lam=1.0, mean_len=15.0, zmax=3000, seed=11)
+    both(contexts, vol, "dilation", "fp32", r)
+
+
+def column_volume(nx, ny, columns, zext):
+    cols = [columns.get(i, []) for i in range(nx * ny)]
+    return CompressedVolume.from_columns(nx, ny, cols, origin=(0.0, 0.0, 0.0), extent=(float(nx), float(ny), zext))
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("n", [3, 4, 8, 9, 24, 25, 200, 600])
+def test_many_intervals(contexts, prec, n):
+    """Columns keeping n separate intervals: within the LDS entries, past
+    them, past the first room (the tile is done again with more), and past what the
+    form takes (the sweeps do the volume)."""
+    vol = column_volume(20, 11, {25: [float(4 * k + j) for k in range(n) for j in (0, 1)],
+                                 97: [4.0 * k + 0.5 + j for k in range(n) for j in (0, 0.25)]}, 4.0 * n)
+    for r in (0.5, 1.2):
+        off, z = both(contexts, vol, "dilation", prec, r)
+        assert np.diff(off).max() == 2 * n
+    both(contexts, vol, "dilation", prec, 9.0)
+
+
+def test_column_of_many_segments(contexts):
+    """More segments in a column than its summary word counts: 70,000 thin
+    ones that the dilation fuses."""
+    n = 70000
+    z = np.arange(2 * n, dtype=np.float64) * 0.5
+    vol = column_volume(9, 3, {4: z.tolist(), 13: [100.0, 40000.0]}, n + 10.0)
+    zlo, zhi = vol.z_range()
+    off, got, _ = contexts[0].morph_host("dilation", "fp64", 2.5, vol.nx, vol.ny, vol.off, vol.z, zlo, zhi)
+    for c, (dx, dy) in {4: (0, 0), 3: (1, 0), 6: (2, 0), 22: (0, 2)}.items():
+        h = np.sqrt(6.25 - dx * dx - dy * dy)
+        assert got[off[c]:off[c + 1]].tolist() == [0.0 - h, z[-1] + h]
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_points_and_touching_segments(contexts, prec):
+    rng = np.random.default_rng(5)
+    cols = {}
+    for c in range(23 * 17):
+        v = np.sort(rng.integers(0, 120, 2 * int(rng.integers(0, 6)))) / 4.0
+        cols[c] = v.tolist()
+    vol = column_volume(23, 17, cols, 40.0)
+    for r in (1.0, 2.5, 5.0, 13.0):
+        both(contexts, vol, "dilation", prec, r)

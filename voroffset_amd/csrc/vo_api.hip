@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "../../include/voroffset_hip.h"
+#include "vo_direct.hpp"
 #include "vo_parity.hpp"
 #include "vo_raster.hpp"
 #include "vo_sweeps.hpp"
@@ -54,6 +55,14 @@ struct Tuning {
 };
 // pass-1 z-sweep form: LDS events per z-slab (denser windows take more slabs)
 // and histogram bins; small enough for ~5 waves per SIMD
+// One-pass form: entries of a lane's interval list kept in LDS.  Small radii
+// leave several intervals in a column and want them there (8 entries against
+// 3: 346 against 423 us for 216 x 310 columns at R = 2, 261 against 302 us for
+// 64 x 48 at R = 4); larger ones leave one or two, and the waves that fit
+// beside each other count (3 entries against 8: 444 against 697 us for 1024^2
+// at R = 16, 537 against 603 us for 512^2 solids at R = 8).
+constexpr int kDirectListSmallR = 8, kDirectListLargeR = 3, kDirectSmallR = 7;
+inline int direct_list(int rint) { return rint <= kDirectSmallR ? kDirectListSmallR : kDirectListLargeR; }
 constexpr int kZECap = 768, kZNB = 512, kZWMax = 64 + 2 * 128, kZWMax8 = 64 + 2 * 256;
 
 template <class T>
@@ -110,6 +119,7 @@ enum Slot {
   kM_SLO, kM_SHI, kM_CHI,                                    // pass-1 block and column summaries
   kX_SCR, kX_N1, kX_N2, kX_LEN, kX_OFF, kX_Z, kX_LENGTH, kX_SEGS, kX_SUM,  // parity metrics
   kV_WORD, kV_TAB, kV_BASE,                // device-side input check
+  kD_COL, kD_AT, kD_BLK, kD_BCNT, kD_TAB,  // one-pass dilation: summaries, H table and block order
   kB_OUT,                                  // + (stage * 3 + kind) * 2 (+1 for z): stage outputs
   kSLOTS = kB_OUT + 4 * 3 * 2
 };
@@ -187,6 +197,13 @@ struct vo_context {
   // with the same radius skips the upload)
   double htab_R = -1;
   const void* htab_at = nullptr;
+  // the same for the one-pass form's table and block order
+  double dtab_R = -1;
+  int dtab_axis = 0;
+  const void* dtab_at = nullptr;
+  int dtab_norder = 0;
+  bool two_pass = false;  // VO_PASS1=zsweep, vo_pass1, vo_autotune: keep to the two sweeps
+  int direct_cap = 24;    // intervals per list of the one-pass form (grows on overflow)
   int64_t spec_out = 0;  // endpoints the next dilation's output is first sized for
   // an input check left to the pass 1 of the operation's first dilation
   // (word == null: none pending); see defer_input_check
@@ -487,6 +504,237 @@ template <class T>
 void enqueue_input_check(vo_context* ctx, const std::vector<vo::InputCheck<T>>& jobs,
                          const std::vector<int64_t>& ncols, const std::vector<int>& job_ids);
 
+// The one-pass form's H table for radius R (entry [adx * W + ady], the
+// differences taken in the order the sweeps' table takes them for this axis)
+// and its blocks in reach, nearest first.
+struct DirectTable {
+  std::vector<double> h;
+  std::vector<int2> order;
+};
+
+DirectTable direct_table(double R, bool along_x) {
+  const int rint = int(std::floor(R)), W = vo::direct_htab_width(rint);
+  const double R2 = R * R;
+  DirectTable t;
+  t.h.resize(size_t(W) * W, std::nan(""));
+  for (int ax = 0; ax <= rint; ++ax)
+    for (int ay = 0; ay <= rint; ++ay) {
+      const double dy = along_x ? ax : ay, ad = along_x ? ay : ax;
+      const double v = R2 - dy * dy - ad * ad;
+      if (v >= 0) t.h[size_t(ax) * W + ay] = std::sqrt(v);
+    }
+  auto gap = [](int d) { return d == 0 ? 0 : vo::kSide * (std::abs(d) - 1) + 1; };
+  const int m = (rint + vo::kSide - 1) / vo::kSide;
+  for (int y = -m; y <= m; ++y)
+    for (int x = -m; x <= m; ++x)
+      if (gap(x) <= rint && gap(y) <= rint && !std::isnan(t.h[size_t(gap(x)) * W + gap(y)])) t.order.push_back(int2{x, y});
+  std::stable_sort(t.order.begin(), t.order.end(), [&](const int2& a, const int2& b) {
+    auto key = [&](const int2& o) {
+      return std::make_pair(gap(o.x) * gap(o.x) + gap(o.y) * gap(o.y), o.x * o.x + o.y * o.y);
+    };
+    return key(a) < key(b);
+  });
+  return t;
+}
+
+// Whether a dilation by `rint` whole dexels takes the one-pass form.
+bool takes_direct(const vo_context* ctx, int rint) {
+  return ctx->pass1_form == 0 && !ctx->force_sweep && !ctx->two_pass && rint <= vo::kDirectMaxR;
+}
+
+template <class T>
+void launch_direct(vo_context* ctx, int rint, const vo::DirectArgs<T>& a, int ntiles) {
+  const dim3 g(blocks_for(ntiles, vo::kDirectWaves)), b(vo::kWave * vo::kDirectWaves);
+  const int W = vo::direct_htab_width(rint);
+  const size_t lds = size_t(W) * W * sizeof(double);
+  if (rint <= kDirectSmallR)
+    hipLaunchKernelGGL((vo::direct_kernel<T, kDirectListSmallR, true>), g, b, lds, ctx->stream, a, ntiles);
+  else if (rint <= vo::kDirectLdsTableMax)
+    hipLaunchKernelGGL((vo::direct_kernel<T, kDirectListLargeR, true>), g, b, lds, ctx->stream, a, ntiles);
+  else
+    hipLaunchKernelGGL((vo::direct_kernel<T, kDirectListLargeR, false>), g, b, 0, ctx->stream, a, ntiles);
+}
+
+// One dilation in one pass (vo_direct.hpp): returns false, with nothing done,
+// where the two sweeps have to take it (no room in the no-alloc scratch, or
+// lists past
+// kDirectMaxList or kGatherRoomBytes).  `chk` is a pending input check (word null:
+// none), done by the summary kernel.
+template <class T>
+bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, const vo::InputCheck<T>& chk, int* chk_word,
+                   int64_t* out_off, int out_z_slot, DevVol& out, double* t1, double* t2) {
+  const int rint = int(std::floor(R));
+  const int nbx = (in.nx + vo::kSide - 1) / vo::kSide, nby = (in.ny + vo::kSide - 1) / vo::kSide;
+  const int64_t ncols = int64_t(in.nx) * in.ny, ntiles = int64_t(nbx) * nby;
+  if (ntiles * vo::kWave > INT32_MAX) return false;
+  const bool along_x = ax.sy == 1;
+  int* status = static_cast<int*>(slot_ptr(ctx, kSTATUS));
+  int64_t* o_start = static_cast<int64_t*>(slot_ptr(ctx, kO_START));
+  int64_t* o_len = static_cast<int64_t*>(slot_ptr(ctx, kO_LEN));
+  int cap = ctx->direct_cap;
+  const int in_lds = direct_list(rint);
+  const int W = vo::direct_htab_width(rint);
+  DirectTable tab;  // outlives its upload (a synchronisation follows)
+  const bool cached = !ctx->arena.on && ctx->dtab_R == R && ctx->dtab_axis == int(along_x) && ctx->dtab_at;
+  if (!cached) tab = direct_table(R, along_x);
+  const size_t hbytes = size_t(W) * W * sizeof(double);
+  int norder = cached ? ctx->dtab_norder : int(tab.order.size());
+  const size_t tbytes = hbytes + size_t(norder) * sizeof(int2);
+  auto list_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * 2 * (c - in_lds) * vo::kWave * sizeof(double); };
+  auto out_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * 2 * c * vo::kWave * sizeof(T); };
+  vo::Ends<T>*col, *blk;
+  uint64_t* at;
+  int *bcnt, *tiles;
+  char* dtab;
+  T* o_z;
+  double* spill;
+  if (ctx->arena.on) {
+    // the sweeps' buffers are reserved already; this form's go inside them
+    size_t used = 0;
+    const Buffer& pool = ctx->arena.slot[kM_LO];
+    bool fits = true;
+    auto take = [&](size_t bytes) {
+      char* p = static_cast<char*>(pool.ptr) + used;
+      used += (bytes + 255) & ~size_t(255);
+      fits = fits && used <= pool.bytes;
+      return p;
+    };
+    col = reinterpret_cast<vo::Ends<T>*>(take(size_t(ntiles) * vo::kWave * sizeof(vo::Ends<T>)));
+    at = reinterpret_cast<uint64_t*>(take(size_t(ntiles) * vo::kWave * sizeof(uint64_t)));
+    blk = reinterpret_cast<vo::Ends<T>*>(take(size_t(ntiles) * sizeof(vo::Ends<T>)));
+    bcnt = reinterpret_cast<int*>(take(size_t(ntiles) * sizeof(int)));
+    tiles = reinterpret_cast<int*>(take(size_t(ntiles + 1) * sizeof(int)));
+    dtab = take(tbytes);
+    const Buffer &lists = ctx->arena.slot[kG_LISTS], &oz = ctx->arena.slot[kO_Z];
+    cap = int(std::min(std::min(size_t(cap), oz.bytes / out_bytes(ntiles, 1)), in_lds + lists.bytes / list_bytes(ntiles, in_lds + 1)));
+    if (!fits || cap < 12) return false;
+    spill = static_cast<double*>(lists.ptr);
+    o_z = static_cast<T*>(oz.ptr);
+  } else {
+    col = static_cast<vo::Ends<T>*>(ws(ctx, kD_COL, size_t(ntiles) * vo::kWave * sizeof(vo::Ends<T>)));
+    at = static_cast<uint64_t*>(ws(ctx, kD_AT, size_t(ntiles) * vo::kWave * sizeof(uint64_t)));
+    blk = static_cast<vo::Ends<T>*>(ws(ctx, kD_BLK, size_t(ntiles) * sizeof(vo::Ends<T>)));
+    bcnt = static_cast<int*>(ws(ctx, kD_BCNT, size_t(ntiles) * sizeof(int)));
+    tiles = static_cast<int*>(ws(ctx, kTILES, size_t(2 * ntiles + 2) * sizeof(int)));
+    dtab = static_cast<char*>(ws(ctx, kD_TAB, tbytes));
+    spill = static_cast<double*>(ws(ctx, kG_LISTS, list_bytes(ntiles, cap)));
+    o_z = static_cast<T*>(ws(ctx, kO_Z, out_bytes(ntiles, cap)));
+  }
+  hipLaunchKernelGGL(vo::reset_words_kernel, dim3(1), dim3(1), 0, ctx->stream, status, tiles, o_len + ncols, chk_word);
+  check(ctx, hipGetLastError(), "reset words");
+  if (!cached || dtab != ctx->dtab_at) {
+    if (cached) tab = direct_table(R, along_x);
+    ctx->dtab_R = -1;  // (until the upload is in the stream)
+    check(ctx, hipMemcpyAsync(dtab, tab.h.data(), hbytes, hipMemcpyHostToDevice, ctx->stream), "upload H table");
+    check(ctx, hipMemcpyAsync(dtab + hbytes, tab.order.data(), tab.order.size() * sizeof(int2), hipMemcpyHostToDevice,
+                              ctx->stream),
+          "upload H table");
+    if (!ctx->arena.on) {
+      ctx->dtab_R = R;
+      ctx->dtab_axis = int(along_x);
+      ctx->dtab_at = dtab;
+      ctx->dtab_norder = norder;
+    }
+  }
+  const T* z = static_cast<const T*>(in.z);
+  check(ctx, hipEventRecord(ctx->ev[0], ctx->stream), "event");
+  {
+    vo::SummaryArgs<T> a{in.nx, in.ny, nbx, nby, in.off, z, col, at, blk, bcnt, chk_word, chk.range, chk.lo, chk.hi};
+    const int64_t grid = int64_t((nbx + vo::kSide - 1) / vo::kSide) * nby;
+    hipLaunchKernelGGL(vo::summary_kernel<T>, dim3(unsigned(grid)), dim3(vo::kWave * vo::kSide), 0, ctx->stream, a);
+    check(ctx, hipGetLastError(), "pass1 launch");
+  }
+  check(ctx, hipEventRecord(ctx->ev[1], ctx->stream), "event");
+  vo::DirectArgs<T> a{in.nx, in.ny, nbx, nby, rint, in.off, z, col, at, blk, bcnt,
+                      reinterpret_cast<const double*>(dtab), reinterpret_cast<const int2*>(dtab + hbytes), norder,
+                      o_z, int64_t(2) * cap * vo::kWave, 0, o_start, o_len, cap, spill, tiles, status, nullptr};
+  int64_t todo = ntiles, done_tiles = 0;  // tiles of this launch, and output regions used by earlier ones
+  int64_t total = -1;
+  bool copied = false;
+  for (;;) {
+    launch_direct<T>(ctx, rint, a, int(todo));
+    check(ctx, hipGetLastError(), "pass2 gather launch");
+    check(ctx, hipEventRecord(ctx->ev[2], ctx->stream), "event");
+    exclusive_scan(ctx, o_len, out_off, ncols + 1);
+    hipLaunchKernelGGL(vo::report_words_kernel, dim3(1), dim3(1), 0, ctx->stream, out_off + ncols, status, a.tile_list,
+                       chk_word, ctx->host_words);
+    check(ctx, hipGetLastError(), "report words");
+    // the CSR copy before the synchronisation, into an output sized like the
+    // last result plus a quarter (see dilate)
+    int64_t spec = 0;
+    if (!ctx->arena.on) {
+      spec = std::max<int64_t>(ctx->spec_out, 16);
+      T* oz = static_cast<T*>(ws(ctx, out_z_slot, size_t(spec) * sizeof(T)));
+      hipLaunchKernelGGL(vo::gather_kernel<T>, dim3(blocks_for(ncols, 256)), dim3(256), 0, ctx->stream, ncols,
+                         static_cast<const T*>(o_z), o_start, o_len, out_off, oz, INT64_MAX, spec);
+      check(ctx, hipGetLastError(), "gather launch");
+    }
+    sync(ctx);
+    const int64_t nfall = int64_t(uint32_t(ctx->host_words[2]));
+    if (nfall == 0) {
+      total = ctx->host_words[0];
+      copied = total <= spec;
+      break;
+    }
+    // lists outgrew their capacity: those tiles again with twice the room
+    // (their output goes past the earlier ones'), up to kGatherRoomBytes
+    if (ctx->arena.on) return false;
+    done_tiles += todo * a.cap;
+    const int c2 = 2 * a.cap;
+    const size_t room = size_t(done_tiles + nfall * c2) * 2 * vo::kWave * sizeof(T) + list_bytes(nfall, c2);
+    if (room > kGatherRoomBytes || c2 > vo::kDirectMaxList) return false;
+    // the output arena may have to move: what it holds comes along
+    if (size_t(done_tiles + nfall * c2) * 2 * vo::kWave * sizeof(T) > ctx->buf[kO_Z].bytes) {
+      Buffer old = ctx->buf[kO_Z];
+      ctx->buf[kO_Z] = Buffer();
+      T* moved = nullptr;
+      try {
+        moved = static_cast<T*>(ws(ctx, kO_Z, size_t(done_tiles + nfall * c2) * 2 * vo::kWave * sizeof(T)));
+        check(ctx, hipMemcpyAsync(moved, old.ptr, size_t(done_tiles) * 2 * vo::kWave * sizeof(T), hipMemcpyDeviceToDevice,
+                                  ctx->stream),
+              "copy");
+        check(ctx, hipStreamSynchronize(ctx->stream), "sync");
+      } catch (...) {
+        (void)hipFree(old.ptr);
+        throw;
+      }
+      check(ctx, hipFree(old.ptr), "hipFree");
+      o_z = moved;
+    }
+    // the list is read by the next launch while it writes the other half
+    int* next = a.tile_list == tiles ? tiles + ntiles + 1 : tiles;
+    a.only = a.tile_list + 1;
+    a.tile_list = next;
+    check(ctx, hipMemsetAsync(next, 0, sizeof(int), ctx->stream), "memset tiles");
+    a.o_z = o_z;
+    a.o_base = done_tiles * 2 * vo::kWave;
+    a.cap = c2;
+    a.garena = int64_t(2) * c2 * vo::kWave;
+    a.spill = static_cast<double*>(ws(ctx, kG_LISTS, list_bytes(nfall, c2)));
+    if (c2 <= 64) ctx->direct_cap = c2;  // the next calls start with the room this one needed
+    todo = nfall;
+  }
+  ctx->last_fallback_tiles = 0;
+  if (t1 || t2) {
+    float ms1 = 0, ms2 = 0;
+    check(ctx, hipEventElapsedTime(&ms1, ctx->ev[0], ctx->ev[1]), "elapsed");
+    check(ctx, hipEventElapsedTime(&ms2, ctx->ev[1], ctx->ev[2]), "elapsed");
+    if (t1) *t1 = ms1;
+    if (t2) *t2 = ms2;
+  }
+  T* oz = static_cast<T*>(ws(ctx, out_z_slot, size_t(std::max<int64_t>(total, 1)) * sizeof(T)));
+  if (!copied) {
+    hipLaunchKernelGGL(vo::gather_kernel<T>, dim3(blocks_for(ncols, 256)), dim3(256), 0, ctx->stream, ncols,
+                       static_cast<const T*>(o_z), o_start, o_len, out_off, oz, INT64_MAX, std::max<int64_t>(total, 0));
+    check(ctx, hipGetLastError(), "gather launch");
+  }
+  if (!ctx->arena.on) ctx->spec_out = total + total / 4;
+  out.z = oz;
+  out.count = total;
+  ctx->last_outputs = total;
+  return true;
+}
+
 // One dilation: `in` -> CSR in (out_off_slot, out_z_slot).
 template <class T>
 DevVol dilate(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int out_z_slot, double* t1,
@@ -520,6 +768,27 @@ DevVol dilate(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int
     check(ctx, hipMemsetAsync(out_off, 0, sizeof(int64_t), ctx->stream), "memset");
     out.z = ws(ctx, out_z_slot, 16);
     return out;
+  }
+  if (takes_direct(ctx, rint)) {
+    if (ctx->arena.on) {
+      // the no-alloc scratch is sized, and a volume refused, by what the two
+      // sweeps need; the one-pass form works inside their buffers
+      const int64_t slots = ncols * ctx->p1_caps;
+      const int64_t nt = int64_t(nx) * ((ny + vo::kGatherTile - 1) / vo::kGatherTile);
+      const int gocap = ocap_for(ctx, rint);
+      ws(ctx, kM_LO, slots * sizeof(T));
+      ws(ctx, kM_HI, slots * sizeof(T));
+      ws(ctx, kM_DY, slots * sizeof(uint16_t));
+      ws(ctx, kM_SLO, size_t(slots / vo::kSlotBlock) * sizeof(T));
+      ws(ctx, kM_SHI, size_t(slots / vo::kSlotBlock) * sizeof(T));
+      ws(ctx, kM_CHI, size_t(ncols) * sizeof(T));
+      ws(ctx, kO_Z, size_t(nt * vo::kGatherTile * (2 * gocap + ctx->p2_cap_per_col)) * sizeof(T));
+      ws(ctx, kTILES, (nt + 1) * sizeof(int));
+      ws(ctx, kG_HTAB, size_t(rint + 1) * vo::htab_width(rint) * sizeof(double));
+      ws(ctx, kG_LISTS, size_t(nt) * 2 * gocap * vo::kWave * sizeof(double));
+    }
+    const vo::InputCheck<T> c{in.off, static_cast<const T*>(in.z), chk_range, chk_lo, chk_hi};
+    if (dilate_direct<T>(ctx, in, R, ax, c, chk_word, out_off, out_z_slot, out, t1, t2)) return out;
   }
   std::vector<double> htab_host;  // outlives the uploads (the gather is followed by a synchronisation)
   int chunk1 = std::min(Shapes<T>::p1_cmax, 32);
@@ -1596,6 +1865,12 @@ void autotune(vo_context* ctx, const vo_volume* sample, int n, const double* rad
   in.off = sample->offsets;
   in.z = sample->z;
   const int forced = ctx->zsweep_events;
+  struct Sweeps {  // the shapes it tunes are the two sweeps'
+    vo_context* c;
+    bool was;
+    ~Sweeps() { c->two_pass = was; }
+  } sweeps{ctx, ctx->two_pass};
+  ctx->two_pass = true;
   for (int i = 0; i < n; ++i) {
     const double R = radii[i];
     if (!(R >= 0) || !std::isfinite(R) || R > 127) fail(ctx, VO_ERR_ARGUMENT, "vo_autotune: radius out of [0, 127]");
@@ -1908,14 +2183,18 @@ void pass1_host(vo_context* ctx, double R, const vo_volume* in, vo_triples* res)
   DevVol v = upload_host<T>(ctx, in, shift);
   // the reference's axis: lines of constant x, swept along y
   const int forced = ctx->axis_forced;
+  const bool two_pass = ctx->two_pass;
   ctx->axis_forced = 0;
+  ctx->two_pass = true;
   try {
     dilate<T>(ctx, v, R, kV3_OFF, kV3_Z, nullptr, nullptr);
   } catch (...) {
     ctx->axis_forced = forced;
+    ctx->two_pass = two_pass;
     throw;
   }
   ctx->axis_forced = forced;
+  ctx->two_pass = two_pass;
   const int64_t n = int64_t(in->nx) * in->ny;
   res->nx = in->nx;
   res->ny = in->ny;
@@ -2006,8 +2285,10 @@ int vo_create(vo_context** out, int device) {
   if (const char* e = std::getenv("VO_BATCH_GRAPH")) ctx->use_graphs = std::string(e) != "0";
   if (const char* e = std::getenv("VO_BATCH_QUEUE")) ctx->batch_queue = std::string(e) == "1";
   if (const char* e = std::getenv("VO_AXIS")) ctx->axis_forced = std::string(e) == "x" ? 1 : (std::string(e) == "y" ? 0 : -1);
-  if (const char* e = std::getenv("VO_PASS1"))
+  if (const char* e = std::getenv("VO_PASS1")) {
     ctx->pass1_form = std::string(e) == "cull" ? 2 : (std::string(e) == "paint" ? 1 : 0);
+    ctx->two_pass = std::string(e) == "zsweep";
+  }
   int rc = guarded(ctx, [&] {
     int n = 0;
     check(ctx, hipGetDeviceCount(&n), "hipGetDeviceCount");

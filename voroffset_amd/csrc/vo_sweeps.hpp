@@ -838,15 +838,57 @@ __device__ void check_column(const InputCheck<T>& g, int64_t c, int job, int* wo
   }
 }
 
-// One volume: a wavefront checks 64 consecutive columns, whose endpoints are
-// one contiguous range, reading it with coalesced loads 64 endpoints at a
-// time, four such loads in flight together (the kernel waits on memory
-// latency, not bandwidth); the columns starting inside each chunk are one
-// 64-bit mask (an
+// The endpoints [S, E) of a wavefront's 64 consecutive columns (this lane's is
+// [s, e) where `has`): read with coalesced loads 64 endpoints at a time, four
+// such loads in flight together (the reader waits on memory latency, not
+// bandwidth); the columns starting inside each chunk are one 64-bit mask (an
 // OR over the lanes), so that an endpoint is compared with the one before it
 // only within its column.  For the ranged operations every endpoint is
 // checked against [lo, hi] (with the columns sorted that is the same as
 // checking their first and last).
+template <class T>
+__device__ __forceinline__ int check_range(const T* z, int64_t S, int64_t E, int64_t s, int64_t e, bool has, int range,
+                                           double lo, double hi) {
+  const int L = lane_id() & (kWave - 1);
+  int bad = 0;
+  T carry = T(0);
+  constexpr int U = 4;
+  for (int64_t sup = S; sup < E; sup += U * kWave) {
+    T vs[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = sup + u * kWave + L;
+      vs[u] = i < E ? z[i] : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t base = sup + u * kWave;
+      if (base >= E) break;  // uniform
+      const int64_t i = base + L;
+      const bool in = i < E;
+      const T v = vs[u];
+      // bit k: an endpoint base + k starts a (non-empty) column
+      const uint64_t mine = (has && s < e && s >= base && s < base + kWave) ? (uint64_t(1) << (s - base)) : 0;
+      uint64_t starts = mine;
+#pragma unroll
+      for (int d = 1; d < kWave; d <<= 1) starts |= __shfl_xor(starts, d);
+      T pv = __shfl_up(v, 1);
+      pv = L == 0 ? carry : pv;
+      const bool first = ((starts >> L) & 1) != 0 || i == S;
+      int b = 0;
+      if (in) {
+        if (!isfinite(double(v)) || (!first && v < pv)) b = kInputMalformed;
+        else if (range && (double(v) < lo || double(v) > hi)) b = kInputOutOfRange;
+      }
+      bad |= b;
+      carry = __shfl(v, kWave - 1);
+    }
+  }
+  return bad;
+}
+
+// One volume: a wavefront checks 64 consecutive columns, whose endpoints are
+// one contiguous range.
 template <class T>
 __global__ __launch_bounds__(256) void check_input_kernel(InputCheck<T> g, int64_t ncols, int* word) {
   const int L = lane_id() & (kWave - 1);
@@ -860,42 +902,7 @@ __global__ __launch_bounds__(256) void check_input_kernel(InputCheck<T> g, int64
   // per-column checks run
   const int last = int(min<int64_t>(ncols - c0, kWave)) - 1;
   const int64_t S = __shfl(s, 0), E = __shfl(e, last);
-  if (ballot(bad != 0) == 0 && E > S) {
-    T carry = T(0);
-    // four chunks of 64 endpoints loaded together (one memory round trip)
-    constexpr int U = 4;
-    for (int64_t sup = S; sup < E; sup += U * kWave) {
-      T vs[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = sup + u * kWave + L;
-        vs[u] = i < E ? g.z[i] : T(0);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t base = sup + u * kWave;
-        if (base >= E) break;  // uniform
-        const int64_t i = base + L;
-        const bool in = i < E;
-        const T v = vs[u];
-        // bit k: an endpoint base + k starts a (non-empty) column
-        const uint64_t mine = (has && s < e && s >= base && s < base + kWave) ? (uint64_t(1) << (s - base)) : 0;
-        uint64_t starts = mine;
-#pragma unroll
-        for (int d = 1; d < kWave; d <<= 1) starts |= __shfl_xor(starts, d);
-        T pv = __shfl_up(v, 1);
-        pv = L == 0 ? carry : pv;
-        const bool first = ((starts >> L) & 1) != 0 || i == S;
-        int b = 0;
-        if (in) {
-          if (!isfinite(double(v)) || (!first && v < pv)) b = kInputMalformed;
-          else if (g.range && (double(v) < g.lo || double(v) > g.hi)) b = kInputOutOfRange;
-        }
-        bad |= b;
-        carry = __shfl(v, kWave - 1);
-      }
-    }
-  }
+  if (ballot(bad != 0) == 0 && E > S) bad |= check_range(g.z, S, E, s, e, has, g.range, g.lo, g.hi);
   if (bad) {
     atomicOr(word, bad);
     atomicMin(word + 1, 0);
