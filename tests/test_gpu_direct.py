@@ -62,6 +62,14 @@ def test_solids(contexts, op, r):
         both(contexts, vol, op, prec, r)
 
 
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("r", [2.0, 5.5, 20.0, 40.0])
+def test_one_wavefront_per_tile(contexts, prec, r):
+    """More tiles than share wavefronts (512): one wavefront each."""
+    vol = synth.poisson_columns(233, 150, lam=5, zmax=600, seed=int(r), z_margin=int(r) + 3)
+    both(contexts, vol, "dilation", prec, r)
+
+
 @pytest.mark.parametrize("r", [100.0, 255.0])
 def test_large_radii(contexts, r):
     vol = synth.poisson_columns(300, 20, lam=1.0, mean_len=15.0, zmax=3000, seed=11)

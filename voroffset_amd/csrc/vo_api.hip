@@ -55,14 +55,20 @@ struct Tuning {
 };
 // pass-1 z-sweep form: LDS events per z-slab (denser windows take more slabs)
 // and histogram bins; small enough for ~5 waves per SIMD
-// One-pass form: entries of a lane's interval list kept in LDS.  Small radii
-// leave several intervals in a column and want them there (8 entries against
-// 3: 346 against 423 us for 216 x 310 columns at R = 2, 261 against 302 us for
-// 64 x 48 at R = 4); larger ones leave one or two, and the waves that fit
-// beside each other count (3 entries against 8: 444 against 697 us for 1024^2
-// at R = 16, 537 against 603 us for 512^2 solids at R = 8).
-constexpr int kDirectListSmallR = 8, kDirectListLargeR = 3, kDirectSmallR = 7;
-inline int direct_list(int rint) { return rint <= kDirectSmallR ? kDirectListSmallR : kDirectListLargeR; }
+// One-pass form: few tiles leave most of the card idle, each a long serial
+// chain: up to 512 of them four wavefronts share a tile (86 x 88 solids at
+// R = 6.4: 400 -> 191 us, 212 x 118 closing at R = 27: 466 -> 171, 64 x 48 at
+// R = 4: 255 -> 228; above, the wavefronts' weaker covers cost more than they
+// give: 216 x 310 at R = 2, 1053 tiles, 340 -> 513).
+constexpr int kDirectSplit = 4, kDirectSplitTiles = 512;
+inline int direct_split(int64_t ntiles) { return ntiles <= kDirectSplitTiles ? kDirectSplit : 1; }
+// Entries of a lane's interval list kept in LDS: the long list where columns
+// keep several intervals (small radii) or LDS does not decide how many waves
+// fit (split tiles), the short one elsewhere.
+constexpr int kDirectListLong = 8, kDirectListShort = 3, kDirectSmallR = 3;
+inline int direct_list(int rint, int split) {
+  return split > 1 || rint <= kDirectSmallR ? kDirectListLong : kDirectListShort;
+}
 constexpr int kZECap = 768, kZNB = 512, kZWMax = 64 + 2 * 128, kZWMax8 = 64 + 2 * 256;
 
 template <class T>
@@ -543,16 +549,24 @@ bool takes_direct(const vo_context* ctx, int rint) {
 }
 
 template <class T>
-void launch_direct(vo_context* ctx, int rint, const vo::DirectArgs<T>& a, int ntiles) {
-  const dim3 g(blocks_for(ntiles, vo::kDirectWaves)), b(vo::kWave * vo::kDirectWaves);
+void launch_direct(vo_context* ctx, int rint, int split, const vo::DirectArgs<T>& a, int ntiles) {
   const int W = vo::direct_htab_width(rint);
-  const size_t lds = size_t(W) * W * sizeof(double);
-  if (rint <= kDirectSmallR)
-    hipLaunchKernelGGL((vo::direct_kernel<T, kDirectListSmallR, true>), g, b, lds, ctx->stream, a, ntiles);
-  else if (rint <= vo::kDirectLdsTableMax)
-    hipLaunchKernelGGL((vo::direct_kernel<T, kDirectListLargeR, true>), g, b, lds, ctx->stream, a, ntiles);
+  const bool lds_table = rint <= vo::kDirectLdsTableMax;
+  const size_t lds = lds_table ? size_t(W) * W * sizeof(double) : 0;
+  auto launch = [&](auto kernel, unsigned grid, int waves) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(vo::kWave * waves), lds, ctx->stream, a, ntiles);
+  };
+  const unsigned grid = blocks_for(ntiles, vo::kDirectWaves);
+  if (split > 1 && lds_table)
+    launch(vo::direct_kernel<T, kDirectListLong, true, kDirectSplit>, unsigned(ntiles), kDirectSplit);
+  else if (split > 1)
+    launch(vo::direct_kernel<T, kDirectListLong, false, kDirectSplit>, unsigned(ntiles), kDirectSplit);
+  else if (rint <= kDirectSmallR)
+    launch(vo::direct_kernel<T, kDirectListLong, true, 1>, grid, vo::kDirectWaves);
+  else if (lds_table)
+    launch(vo::direct_kernel<T, kDirectListShort, true, 1>, grid, vo::kDirectWaves);
   else
-    hipLaunchKernelGGL((vo::direct_kernel<T, kDirectListLargeR, false>), g, b, 0, ctx->stream, a, ntiles);
+    launch(vo::direct_kernel<T, kDirectListShort, false, 1>, grid, vo::kDirectWaves);
 }
 
 // One dilation in one pass (vo_direct.hpp): returns false, with nothing done,
@@ -572,7 +586,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   int64_t* o_start = static_cast<int64_t*>(slot_ptr(ctx, kO_START));
   int64_t* o_len = static_cast<int64_t*>(slot_ptr(ctx, kO_LEN));
   int cap = ctx->direct_cap;
-  const int in_lds = direct_list(rint);
+  const int split = direct_split(ntiles), in_lds = direct_list(rint, split);
   const int W = vo::direct_htab_width(rint);
   DirectTable tab;  // outlives its upload (a synchronisation follows)
   const bool cached = !ctx->arena.on && ctx->dtab_R == R && ctx->dtab_axis == int(along_x) && ctx->dtab_at;
@@ -580,7 +594,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   const size_t hbytes = size_t(W) * W * sizeof(double);
   int norder = cached ? ctx->dtab_norder : int(tab.order.size());
   const size_t tbytes = hbytes + size_t(norder) * sizeof(int2);
-  auto list_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * 2 * (c - in_lds) * vo::kWave * sizeof(double); };
+  auto list_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * split * 2 * (c - in_lds) * vo::kWave * sizeof(double); };
   auto out_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * 2 * c * vo::kWave * sizeof(T); };
   vo::Ends<T>*col, *blk;
   uint64_t* at;
@@ -652,7 +666,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   int64_t total = -1;
   bool copied = false;
   for (;;) {
-    launch_direct<T>(ctx, rint, a, int(todo));
+    launch_direct<T>(ctx, rint, split, a, int(todo));
     check(ctx, hipGetLastError(), "pass2 gather launch");
     check(ctx, hipEventRecord(ctx->ev[2], ctx->stream), "event");
     exclusive_scan(ctx, o_len, out_off, ncols + 1);

@@ -25,9 +25,17 @@ constexpr int kDirectWaves = 4;        // tiles (wavefronts) per workgroup: they
 constexpr int kDirectLdsTableMax = 31; // largest radius whose H table is staged in LDS
 constexpr int kDirectMaxR = 255;       // largest radius this form takes
 constexpr int kDirectMaxList = 512;    // longest list it grows to; the sweeps take volumes that need more
-constexpr int kRecs = 3 * kWave;       // segments waiting to be united, per wavefront
+// Sizes that go with the LDS entries of a lane's list: segments and columns
+// that may wait, and the segments worth a drain between blocks.  With a short
+// list (large radii) the waves that fit count, and early drains keep the cover
+// fresh; with a long one (small radii) fewer drains do.
+template <int kList>
+struct DirectShape {
+  static constexpr bool kSmallR = kList > 4;
+  static constexpr int kRecs = kSmallR ? 192 : 160, kPend = kSmallR ? 128 : 96, kDrainAt = kSmallR ? 64 : 24;
+  static_assert(kDrainAt + 2 * kWave <= kRecs, "a block's first and last segments fit beside what waits");
+};
 constexpr int kHeld = 2;               // runs a lane may hold back before they meet its list
-constexpr int kDrainAt = 48;           // segments worth a drain between blocks
 constexpr int kAhead = 4;              // segments whose growths are read together
 constexpr int kCommon = 6;             // intervals of the tile's common cover the segment test looks at
 
@@ -267,16 +275,25 @@ __device__ __forceinline__ void lds_order() {
 
 template <class T, int kList>
 struct DirectSmem {
+  static constexpr int kRecs = DirectShape<kList>::kRecs, kPend = DirectShape<kList>::kPend;
   double list[2][kList][kWave];  // the lanes' lists, first kList entries ([lower, upper][entry][lane])
   double held[2][kHeld][kWave];  // runs on their way to the lists
   T rz[kRecs][2];           // waiting segments
   int rc[kRecs];            // and their column: (x - tile x + 1024) | 8 (y - tile y + 1024) << 16
   double cm[kCommon][2];    // common cover of the tile
+  uint64_t pw[kPend];       // columns whose inner segments are still to be looked at: start and count
+  int pc[kPend];            // and their place, as in rc
 };
 
-// One tile of 8 x 8 output columns, one lane each.
-template <class T, int kList>
-__device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, DirectSmem<T, kList>& sm, const double* htab) {
+// One tile of 8 x 8 output columns, one lane each.  With kSplit > 1 as many
+// wavefronts share the tile: each unites its part of the source columns, and
+// the first one unites the parts (`sm` is the first one's memory, the others'
+// follow it).
+template <class T, int kList, int kSplit>
+__device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, DirectSmem<T, kList>* sms, int part,
+                            const double* htab) {
+  DirectSmem<T, kList>& sm = sms[part];
+  constexpr int kRecs = DirectShape<kList>::kRecs, kPend = DirectShape<kList>::kPend, kDrainAt = DirectShape<kList>::kDrainAt;
   const int L = threadIdx.x & (kWave - 1);
   const int lx = L % kSide, ly = L / kSide;
   const int tx = tile % g.nbx, ty = tile / g.nbx;
@@ -296,7 +313,7 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
   using LdsDouble = __attribute__((address_space(3))) double;
   using GlobalDouble = __attribute__((address_space(1))) double;
   LdsDouble* const lds = (LdsDouble*)&sm.list[0][0][L];
-  GlobalDouble* const far = (GlobalDouble*)(g.spill + slot * (2 * int64_t(cap - kList) * kWave) + L);
+  GlobalDouble* const far = (GlobalDouble*)(g.spill + (slot * kSplit + part) * (2 * int64_t(cap - kList) * kWave) + L);
   auto get = [&](int end, int i) -> double {
     if (i < kList) return lds[(end * kList + i) * kWave];
     return far[(end * (cap - kList) + (i - kList)) * kWave];
@@ -523,53 +540,93 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
     }
     lds_order();
   };
-  // The segments of source block (bx, by) that may change some lane, kept for
-  // the next drain: one lane per source column (those with `take`), tested
-  // against the first `nc` common intervals.
-  auto block = [&](int bx, int by, bool take, int drain_at, int nc) {
-    // which common interval holds [s, e] (-1: none)
-    auto covered = [&](double s, double e) {
-      int m = -1;
-      for (int i = 0; i < nc; ++i) {
-        const double P = sm.cm[i][0], Q = sm.cm[i][1];
-        m = (s >= P && e <= Q) ? i : m;
-      }
-      return m;
-    };
+  int npend = 0;
+  // which of the first nc common intervals holds [s, e] (-1: none)
+  auto covered = [&](int nc, double s, double e) {
+    int m = -1;
+    for (int i = 0; i < nc; ++i) {
+      const double P = sm.cm[i][0], Q = sm.cm[i][1];
+      m = (s >= P && e <= Q) ? i : m;
+    }
+    return m;
+  };
+  auto keep = [&](bool add, T a, T b, int code) {
+    const uint64_t mask = ballot(add);
+    if (add) {
+      const int q = nrec + count_below(mask);
+      sm.rz[q][0] = a;
+      sm.rz[q][1] = b;
+      sm.rc[q] = code;
+    }
+    nrec += popc(mask);
+  };
+  // Source block (bx, by): one lane per source column (those with `take`).  A
+  // column's first and last segment wait for the next drain where they are
+  // not inside one of the first `nc` common intervals; if it has more, and
+  // they may not all be inside, the column waits to be looked at.
+  auto block = [&](int bx, int by, bool take, int nc) {
     const int cx = bx * kSide + lx, cy = by * kSide + ly;
     const int64_t slot = (int64_t(by) * g.nbx + bx) * kWave + L;
     const Ends<T> r = g.col[slot];
     const uint64_t word = g.at[slot];
-    int64_t s = int64_t(word & ((uint64_t(1) << 48) - 1));
-    int count = int(word >> 48);
-    if (ballot(count == kCountMany) != 0) {
-      if (count == kCountMany) count = int(min<int64_t>((g.off[int64_t(cy) * g.nx + cx + 1] - s) / 2, INT32_MAX));
-    }
     // the column's largest growth on any output column of the tile
     const int gx = gap(cx, tx * kSide, tx * kSide + kSide - 1), gy = gap(cy, ty * kSide, ty * kSide + kSide - 1);
     const double h = htab[min(gx, W - 1) * W + min(gy, W - 1)];
+    const int count = int(word >> 48);
     const bool live = take && count > 0 && h == h;
-    const int m0 = live ? covered(double(r.lo0) - h, double(r.hi0) + h) : 0;
-    const int m1 = live ? covered(double(r.lo1) - h, double(r.hi1) + h) : 0;
+    const int m0 = live ? covered(nc, double(r.lo0) - h, double(r.hi0) + h) : 0;
+    const int m1 = live ? covered(nc, double(r.lo1) - h, double(r.hi1) + h) : 0;
     const int code = (cx - tx * kSide + 1024) | (cy - ty * kSide + 1024) << 19;
-    auto keep = [&](bool add, T a, T b) {
-      const uint64_t mask = ballot(add);
-      if (add) {
-        const int q = nrec + count_below(mask);
-        sm.rz[q][0] = a;
-        sm.rz[q][1] = b;
-        sm.rc[q] = code;
+    keep(m0 < 0, r.lo0, r.hi0, code);
+    keep(m1 < 0 && count > 1, r.lo1, r.hi1, code);
+    const bool inner = live && count > 2 && !(m0 >= 0 && m0 == m1);
+    const uint64_t mask = ballot(inner);
+    if (inner) {
+      const int q = npend + count_below(mask);
+      sm.pw[q] = word;
+      sm.pc[q] = code;
+    }
+    npend += popc(mask);
+  };
+  // The last `m` waiting columns, one per lane: their segments between the
+  // first and the last that may change some lane wait for a drain, which
+  // follows where `drain_at` or more do.
+  auto columns = [&](int m, int drain_at, int nc) {
+    lds_order();
+    const bool mine = L < m;
+    const int q = npend - m + L;
+    const uint64_t word = mine ? sm.pw[q] : 0;
+    const int code = mine ? sm.pc[q] : 1024 | 1024 << 19;
+    npend -= m;
+    int64_t s = int64_t(word & ((uint64_t(1) << 48) - 1));
+    int count = int(word >> 48);
+    const int px = (code & 0xffff) - 1024, py = (code >> 19) - 1024;  // place relative to the tile
+    if (ballot(count == kCountMany) != 0) {
+      if (count == kCountMany) {
+        const int64_t c = int64_t(ty * kSide + py) * g.nx + tx * kSide + px;
+        count = int(min<int64_t>((g.off[c + 1] - s) / 2, INT32_MAX));
       }
-      nrec += popc(mask);
-    };
-    keep(m0 < 0, r.lo0, r.hi0);
-    keep(m1 < 0 && count > 1, r.lo1, r.hi1);
-    // The segments between the first and the last, from the end that is not
-    // covered towards the other one, until a segment is inside the common
-    // interval that holds the other end (sorted columns: so is the rest).
-    int left = live && count > 2 && !(m0 >= 0 && m0 == m1) ? count - 2 : 0;
-    const bool back = m0 >= 0 && m1 < 0;
-    const int stop_at = back ? m0 : m1;
+    }
+    double h = 0;
+    int left = 0, stop_at = 0;
+    bool back = false;
+    if (m > 0) {
+      h = htab[gap(px, 0, kSide - 1) * W + gap(py, 0, kSide - 1)];
+      T r[4] = {T(0), T(0), T(0), T(0)};
+      if (mine) {
+        r[0] = g.z[s];
+        r[1] = g.z[s + 1];
+        r[2] = g.z[s + 2 * int64_t(count) - 2];
+        r[3] = g.z[s + 2 * int64_t(count) - 1];
+      }
+      const int m0 = covered(nc, double(r[0]) - h, double(r[1]) + h), m1 = covered(nc, double(r[2]) - h, double(r[3]) + h);
+      // From the end that is not covered towards the other one, until a
+      // segment is inside the common interval that holds the other end
+      // (sorted columns: so is the rest).
+      left = mine && !(m0 >= 0 && m0 == m1) ? count - 2 : 0;
+      back = m0 >= 0 && m1 < 0;
+      stop_at = back ? m0 : m1;
+    }
     // U segments of a column per round trip, the next ones loaded while these
     // are looked at
     constexpr int U = 2;
@@ -600,13 +657,17 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const bool here = j0 + u < left;
-        const int m = here ? covered(double(ta[u]) - h, double(tb[u]) + h) : 0;
-        keep(m < 0, ta[u], tb[u]);
+        const int m = here ? covered(nc, double(ta[u]) - h, double(tb[u]) + h) : 0;
+        keep(m < 0, ta[u], tb[u], code);
         left = here && m >= 0 && m == stop_at ? 0 : left;
       }
     }
   };
 
+  // With kSplit > 1 a wavefront takes its share of the own block's columns
+  // (the first stage's are everyone's: without that cover the others' segments
+  // would all stay) and of the other blocks.
+  const bool mine = kSplit == 1 || ((lx >> 1) + (ly >> 1) * (kSplit == 8 ? 5 : 1)) % kSplit == part;
   const int first_mask = rint >= 12 ? 3 : (rint >= 4 ? 1 : 0), first_at = rint >= 12 ? 2 : 0;
   for (int g0 = 0; g0 < g.norder; g0 += kWave) {
     // 64 blocks at a time, one lane each: their summaries
@@ -622,22 +683,28 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
     uint64_t todo = ballot(bc > 0);
     // the tile's own block goes first, and of it first a sixteenth or a
     // quarter of its columns, which cover most of what the others have
+    uint64_t share = ~uint64_t(0);
+    if constexpr (kSplit > 1) {
+      share = 0;
+      for (int i = 0; i < kWave; i += kSplit) share |= uint64_t(1) << i;
+      share <<= part;
+    }
     int own = g0 == 0 && (todo & 1) ? 2 : 0;
-    todo &= g0 == 0 ? ~uint64_t(1) : ~uint64_t(0);
+    bool sharing = own > 0;
+    todo &= g0 == 0 ? share & ~uint64_t(1) : share;
     bool fresh = true;
     const bool end = g0 + kWave >= g.norder;  // what is left waiting goes with the last group
-    while (own > 0 || todo != 0 || (end && nrec > 0)) {
-      int drain_at = kDrainAt;
-      bool take = true, reached = active;
+    while (own > 0 || todo != 0 || (end && nrec + npend > 0)) {
+      bool take = true, reached = active, now = false, visit = own > 0;
       int ux = tx, uy = ty;
       if (own > 0) {
         take = (((lx - first_at) | (ly - first_at)) & first_mask) == 0;
         take = take == (own == 2);
+        if constexpr (kSplit > 1) take = take && ((own == 2 && first_mask != 0) || mine);
         --own;
-        drain_at = 1;
+        now = true;
       } else if (todo == 0) {
-        take = false;
-        drain_at = 1;
+        now = true;
       } else {
         if (fresh) {
           // blocks inside the first and last intervals of every lane, 64 at once
@@ -665,6 +732,7 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
         // the block against each lane it reaches, at the lane's own distance
         const int gx = gap(x, ux * kSide, ux * kSide + kSide - 1), gy = gap(y, uy * kSide, uy * kSide + kSide - 1);
         const double h = htab[min(gx, W - 1) * W + min(gy, W - 1)];
+        visit = true;
         reached = active && h == h;
         const bool low = u.lo0 - h >= flo;
         const bool in = (low && u.hi1 + h <= fhi) || (u.lo0 - h >= elo && u.hi1 + h <= ehi) ||
@@ -673,7 +741,52 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
       }
       if (old) common();
       // (a lane that has no list yet is covered by nothing)
-      block(ux, uy, take, drain_at, ballot(reached && n == 0) != 0 ? 0 : ncm);
+      const int nc = ballot(reached && n == 0) != 0 ? 0 : ncm;
+      if (visit) block(ux, uy, take, nc);
+
+      const int m = now || npend > kPend - kWave ? min(npend, kWave) : 0;
+      // (the waiting columns are of several blocks: any lane without a list counts)
+      columns(m, now ? 1 : kDrainAt, ballot(active && n == 0) != 0 ? 0 : ncm);
+      if constexpr (kSplit > 1) {
+        // the own block done, the wavefronts' first and last intervals go to
+        // all of them: with a part of the cover each, the blocks to come
+        // would cost every wavefront what they cost one alone
+        if (sharing && own == 0) {
+          sharing = false;
+          sm.held[0][0][L] = flo;
+          sm.held[0][1][L] = elo;
+          sm.held[1][0][L] = fhi;
+          sm.held[1][1][L] = ehi;
+          __syncthreads();
+          for (int w = 1; w < kSplit; ++w) {
+            const DirectSmem<T, kList>& o = sms[(part + w) % kSplit];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const double s = o.held[0][i][L], e = o.held[1][i][L];
+              if (active && ok && s <= e && (s < flo || e > fhi) && (s < elo || e > ehi)) unite_slow(s, e);
+            }
+          }
+          old = true;
+          __syncthreads();
+        }
+      }
+    }
+  }
+  if constexpr (kSplit > 1) {
+    settle();
+    sm.rc[L] = ok ? n : -1;  // the list's length, where nothing waits any more
+    __syncthreads();
+    if (part != 0) return;
+    for (int w = 1; w < kSplit; ++w) {
+      const int nw = sms[w].rc[L];
+      ok = nw < 0 ? 0 : ok;
+      const GlobalDouble* const fw = (const GlobalDouble*)(g.spill + (slot * kSplit + w) * (2 * int64_t(cap - kList) * kWave) + L);
+      for (int i = 0; ballot(ok && i < nw) != 0; ++i) {
+        if (!ok || i >= nw) continue;
+        const double s = i < kList ? sms[w].list[0][i][L] : double(fw[(i - kList) * kWave]);
+        const double e = i < kList ? sms[w].list[1][i][L] : double(fw[(cap - kList + i - kList) * kWave]);
+        if ((s < flo || e > fhi) && (s < elo || e > ehi)) unite_slow(s, e);
+      }
     }
   }
   if (ballot(active && ok == 0) != 0) {
@@ -704,21 +817,26 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
 
 extern __shared__ double vo_direct_htab[];
 
-template <class T, int kList, bool kLdsTable>
-__global__ __launch_bounds__(kWave* kDirectWaves, kList > 4 ? 2 : 4) void direct_kernel(DirectArgs<T> g, int ntiles) {
-  __shared__ DirectSmem<T, kList> sm[kDirectWaves];
+template <class T, int kList, bool kLdsTable, int kSplit>
+__global__ __launch_bounds__(kWave* (kSplit > 1 ? kSplit : kDirectWaves), kSplit > 1 || kList > 4 ? 2 : 4) void direct_kernel(
+    DirectArgs<T> g, int ntiles) {
+  constexpr int kWaves = kSplit > 1 ? kSplit : kDirectWaves;
+  __shared__ DirectSmem<T, kList> sm[kWaves];
   const double* htab = g.htab;
   if constexpr (kLdsTable) {
     const int W = direct_htab_width(g.rint);
-    for (int i = threadIdx.x; i < W * W; i += kWave * kDirectWaves) vo_direct_htab[i] = g.htab[i];
+    for (int i = threadIdx.x; i < W * W; i += kWave * kWaves) vo_direct_htab[i] = g.htab[i];
     __syncthreads();
     htab = vo_direct_htab;
   }
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int64_t i = xcd_tile(blockIdx.x, gridDim.x) * kDirectWaves + w;
-  if (i >= ntiles) return;
+  const int64_t b = xcd_tile(blockIdx.x, gridDim.x), i = kSplit > 1 ? b : b * kDirectWaves + w;
+  if (i >= ntiles) return;  // (a split tile's wavefronts all stay)
   const int tile = g.only ? g.only[i] : int(i);
-  direct_tile<T, kList>(g, tile, i, sm[w], htab);
+  if constexpr (kSplit > 1)
+    direct_tile<T, kList, kSplit>(g, tile, i, sm, w, htab);
+  else
+    direct_tile<T, kList, 1>(g, tile, i, sm + w, 0, htab);
 }
 
 }  // namespace vo
