@@ -553,20 +553,39 @@ void launch_direct(vo_context* ctx, int rint, int split, const vo::DirectArgs<T>
   const int W = vo::direct_htab_width(rint);
   const bool lds_table = rint <= vo::kDirectLdsTableMax;
   const size_t lds = lds_table ? size_t(W) * W * sizeof(double) : 0;
-  auto launch = [&](auto kernel, unsigned grid, int waves) {
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(vo::kWave * waves), lds, ctx->stream, a, ntiles);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned(ntiles)), dim3(vo::kWave * split), lds, ctx->stream, a);
   };
-  const unsigned grid = blocks_for(ntiles, vo::kDirectWaves);
   if (split > 1 && lds_table)
-    launch(vo::direct_kernel<T, kDirectListLong, true, kDirectSplit>, unsigned(ntiles), kDirectSplit);
+    launch(vo::direct_kernel<T, kDirectListLong, true, kDirectSplit>);
   else if (split > 1)
-    launch(vo::direct_kernel<T, kDirectListLong, false, kDirectSplit>, unsigned(ntiles), kDirectSplit);
+    launch(vo::direct_kernel<T, kDirectListLong, false, kDirectSplit>);
   else if (rint <= kDirectSmallR)
-    launch(vo::direct_kernel<T, kDirectListLong, true, 1>, grid, vo::kDirectWaves);
+    launch(vo::direct_kernel<T, kDirectListLong, true, 1>);
   else if (lds_table)
-    launch(vo::direct_kernel<T, kDirectListShort, true, 1>, grid, vo::kDirectWaves);
+    launch(vo::direct_kernel<T, kDirectListShort, true, 1>);
   else
-    launch(vo::direct_kernel<T, kDirectListShort, false, 1>, grid, vo::kDirectWaves);
+    launch(vo::direct_kernel<T, kDirectListShort, false, 1>);
+}
+
+// Radius class of a batched job in the one-pass form: the kernel it takes.
+int direct_class(int rint) { return rint <= kDirectSmallR ? 0 : (rint <= vo::kDirectLdsTableMax ? 1 : 2); }
+
+// The batched form over the n global tiles from t0 on, all of class c, radii
+// up to max_rint.
+template <class T>
+void launch_direct_batch(vo_context* ctx, int c, int max_rint, const vo::DirectArgs<T>* jobs, const int64_t* tile_base,
+                         int njobs, int64_t t0, int64_t n) {
+  const int W = vo::direct_htab_width(max_rint);
+  auto launch = [&](auto kernel, size_t lds) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned(n)), dim3(vo::kWave), lds, ctx->stream, jobs, tile_base, njobs, t0, n);
+  };
+  if (c == 0)
+    launch(vo::direct_batch_kernel<T, kDirectListLong, true>, size_t(W) * W * sizeof(double));
+  else if (c == 1)
+    launch(vo::direct_batch_kernel<T, kDirectListShort, true>, size_t(W) * W * sizeof(double));
+  else
+    launch(vo::direct_batch_kernel<T, kDirectListShort, false>, 0);
 }
 
 // One dilation in one pass (vo_direct.hpp): returns false, with nothing done,
@@ -1281,7 +1300,8 @@ struct ProgStep {
   int off_slot = 0, z_slot = 0;
   int64_t* off = nullptr;  // output CSR over the step's columns (absolute into z)
   void* z = nullptr;
-  size_t t0 = 0, t1 = 0, t2 = 0, t3 = 0;  // table offsets in the blob
+  std::vector<int64_t> sum_base;  // one-pass dilation: the summary kernel's workgroups
+  size_t t0 = 0, t1 = 0, t2 = 0, t3 = 0, t4 = 0;  // table offsets in the blob
   int64_t cls_t0[3] = {0, 0, 0}, cls_t1[3] = {0, 0, 0};
   int cls_rmax[3] = {0, 0, 0};
 };
@@ -1348,6 +1368,10 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   }
   if (n == 0) return;
   const int tsize = int(sizeof(T));
+  // the dilations' form: one pass, or the two sweeps where a switch asks for
+  // them (batchable() leaves out the radii neither takes)
+  const bool direct = takes_direct(ctx, 0) && !ctx->batch_queue;
+  auto class_of = [&](double r) { return direct ? direct_class(int(std::floor(r))) : radius_class(int(std::floor(r))); };
   std::vector<char> inprog(n, 0);
   for (int j = 0; j < n; ++j) inprog[j] = batchable(ctx, op[j], R[j], vol[j].nx, vol[j].ny, tsize) ? 1 : 0;
 
@@ -1380,7 +1404,8 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   // 2. the program's steps, with every output bounded
   int ocap = 0;
   for (int j = 0; j < n; ++j)
-    if (inprog[j] && op[j] != VO_OP_NOOP) ocap = std::max(ocap, ocap_for(ctx, int(std::floor(R[j]))));
+    if (inprog[j] && op[j] != VO_OP_NOOP)
+      ocap = std::max(ocap, direct ? ctx->direct_cap : ocap_for(ctx, int(std::floor(R[j]))));
   struct Cur {
     int nx, ny;
     int64_t E;
@@ -1398,7 +1423,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
       if (st.jobs.empty()) continue;
       if (kind == kStepDilate)  // grouped by radius class: one range of tiles per class
         std::stable_sort(st.jobs.begin(), st.jobs.end(), [&](int a, int b) {
-          return radius_class(int(std::floor(R[a]))) < radius_class(int(std::floor(R[b])));
+          return class_of(R[a]) < class_of(R[b]);
         });
       const int K = int(st.jobs.size());
       st.col_base.assign(K + 1, 0);
@@ -1418,7 +1443,11 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
         st.zcap += c.E;
         if (kind == kStepDilate) {
           const Axis ax = axis_for(ctx, c.nx, c.ny);
-          st.tile_base[k + 1] = st.tile_base[k] + int64_t(ax.nx) * ((ax.ny + vo::kGatherTile - 1) / vo::kGatherTile);
+          const int64_t nbx = (c.nx + vo::kSide - 1) / vo::kSide, nby = (c.ny + vo::kSide - 1) / vo::kSide;
+          st.tile_base[k + 1] = st.tile_base[k] + (direct ? nbx * nby
+                                                          : int64_t(ax.nx) * ((ax.ny + vo::kGatherTile - 1) / vo::kGatherTile));
+          if (k == 0) st.sum_base.assign(K + 1, 0);
+          st.sum_base[k + 1] = st.sum_base[k] + (nbx + vo::kSide - 1) / vo::kSide * nby;
         }
       }
       st.C = st.col_base[K];
@@ -1438,7 +1467,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   // 3. workspace, sized for the largest step (steps run one after the other)
   const int caps = ctx->p1_caps;
   const int64_t garena = int64_t(vo::kGatherTile) * 2 * ocap;
-  const int64_t list_tile = 2 * int64_t(ocap) * vo::kWave;
+  const int64_t list_tile = 2 * int64_t(direct ? ocap - kDirectListShort : ocap) * vo::kWave;
   for (auto& st : steps) {
     st.off = static_cast<int64_t*>(ws(ctx, st.off_slot, size_t(st.C + 1) * sizeof(int64_t)));
     st.z = ws(ctx, st.z_slot, size_t(std::max<int64_t>(st.zcap, 1)) * sizeof(T));
@@ -1457,7 +1486,18 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   int32_t* m_cnt = nullptr;
   int64_t* o_start = nullptr;
   double* lists = nullptr;
-  if (maxDilC > 0) {
+  vo::Ends<T>*d_col = nullptr, *d_blk = nullptr;
+  uint64_t* d_at = nullptr;
+  int* d_bcnt = nullptr;
+  if (maxDilC > 0 && direct) {
+    d_col = static_cast<vo::Ends<T>*>(ws(ctx, kD_COL, size_t(maxNT) * vo::kWave * sizeof(vo::Ends<T>)));
+    d_at = static_cast<uint64_t*>(ws(ctx, kD_AT, size_t(maxNT) * vo::kWave * sizeof(uint64_t)));
+    d_blk = static_cast<vo::Ends<T>*>(ws(ctx, kD_BLK, size_t(maxNT) * sizeof(vo::Ends<T>)));
+    d_bcnt = static_cast<int*>(ws(ctx, kD_BCNT, size_t(maxNT) * sizeof(int)));
+    o_z = static_cast<T*>(ws(ctx, kO_Z, size_t(maxNT) * garena * sizeof(T)));
+    o_start = static_cast<int64_t*>(ws(ctx, kO_START, size_t(maxDilC) * sizeof(int64_t)));
+    lists = static_cast<double*>(ws(ctx, kG_LISTS, size_t(maxNT) * list_tile * sizeof(double)));
+  } else if (maxDilC > 0) {
     m_lo = static_cast<T*>(ws(ctx, kM_LO, size_t(maxDilC) * caps * sizeof(T)));
     m_hi = static_cast<T*>(ws(ctx, kM_HI, size_t(maxDilC) * caps * sizeof(T)));
     m_dy = static_cast<uint16_t*>(ws(ctx, kM_DY, size_t(maxDilC) * caps * sizeof(uint16_t)));
@@ -1490,7 +1530,46 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   std::vector<DevVol> v = vol;  // each job's current volume as the steps go
   for (auto& st : steps) {
     const int K = int(st.jobs.size());
-    if (st.kind == kStepDilate) {
+    if (st.kind == kStepDilate && direct) {
+      std::vector<double> htab;
+      std::vector<int2> order;
+      std::vector<vo::SummaryArgs<T>> a1(K);
+      std::vector<vo::DirectArgs<T>> a2(K);
+      for (int k = 0; k < K; ++k) {
+        const int j = st.jobs[k];
+        const DevVol& in = v[j];
+        const int rint = int(std::floor(R[j])), c = direct_class(rint);
+        const int nbx = (in.nx + vo::kSide - 1) / vo::kSide, nby = (in.ny + vo::kSide - 1) / vo::kSide;
+        const int64_t cb = st.col_base[k], tb = st.tile_base[k];
+        const DirectTable t = direct_table(R[j], axis_for(ctx, in.nx, in.ny).sy == 1);
+        // (the tables' places stay relative until the blob's address is known)
+        const size_t hat = htab.size() * sizeof(double), oat = order.size() * sizeof(int2);
+        htab.insert(htab.end(), t.h.begin(), t.h.end());
+        order.insert(order.end(), t.order.begin(), t.order.end());
+        const T* z = static_cast<const T*>(in.z);
+        a1[k] = vo::SummaryArgs<T>{in.nx, in.ny, nbx, nby, in.off, z, d_col + tb * vo::kWave, d_at + tb * vo::kWave,
+                                   d_blk + tb, d_bcnt + tb, nullptr, 0, 0.0, 0.0};
+        a2[k] = vo::DirectArgs<T>{in.nx, in.ny, nbx, nby, rint, in.off, z, a1[k].col, a1[k].at, a1[k].blk, a1[k].bcnt,
+                                  reinterpret_cast<const double*>(hat), reinterpret_cast<const int2*>(oat),
+                                  int(t.order.size()), o_z, garena, tb * garena, o_start + cb, len + cb, ocap,
+                                  lists + tb * list_tile, nullptr, status + j, nullptr};
+        if (st.cls_t1[c] == 0) st.cls_t0[c] = st.tile_base[k];
+        st.cls_t1[c] = st.tile_base[k + 1];
+        st.cls_rmax[c] = std::max(st.cls_rmax[c], rint);
+        v[j].off = st.off + cb;
+        v[j].z = st.z;
+      }
+      st.t3 = blob.put(htab);
+      const size_t order_at = blob.put(order);
+      for (auto& a : a2) {
+        a.htab = reinterpret_cast<const double*>(st.t3 + reinterpret_cast<size_t>(a.htab));
+        a.order = reinterpret_cast<const int2*>(order_at + reinterpret_cast<size_t>(a.order));
+      }
+      st.t0 = blob.put(a1);
+      st.t1 = blob.put(a2);
+      st.t2 = blob.put(st.tile_base);
+      st.t4 = blob.put(st.sum_base);
+    } else if (st.kind == kStepDilate) {
       std::vector<double> radii(K), htab;
       std::vector<int64_t> hbase(K, 0);
       for (int k = 0; k < K; ++k) {
@@ -1554,12 +1633,28 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   // the H-table pointers of the pass-2 tables are blob offsets: make them device addresses
   for (auto& st : steps) {
     if (st.kind != kStepDilate) continue;
+    if (direct) {
+      auto* a2 = reinterpret_cast<vo::DirectArgs<T>*>(blob.host.data() + st.t1);
+      for (size_t k = 0; k < st.jobs.size(); ++k) {
+        a2[k].htab = reinterpret_cast<const double*>(dblob + reinterpret_cast<size_t>(a2[k].htab));
+        a2[k].order = reinterpret_cast<const int2*>(dblob + reinterpret_cast<size_t>(a2[k].order));
+      }
+      continue;
+    }
     auto* a2 = reinterpret_cast<vo::Pass2GArgs<T>*>(blob.host.data() + st.t1);
     for (size_t k = 0; k < st.jobs.size(); ++k)
       a2[k].htab = reinterpret_cast<const double*>(dblob + reinterpret_cast<size_t>(a2[k].htab));
   }
 
   // 5. the program: enqueued, captured or replayed
+  auto finish_dilation = [&](const ProgStep& st) {  // output lengths to CSR
+    exclusive_scan(ctx, len, st.off, st.C + 1);
+    if (st.C > 0) {  // (a step over empty grids only has its one offset)
+      hipLaunchKernelGGL(vo::gather_kernel<T>, dim3(blocks_for(st.C, 256)), dim3(256), 0, ctx->stream, st.C,
+                         static_cast<const T*>(o_z), o_start, len, st.off, static_cast<T*>(st.z), INT64_MAX, INT64_MAX);
+      check(ctx, hipGetLastError(), "gather launch");
+    }
+  };
   auto enqueue = [&] {
     fill_words(ctx, status, n, 0);
     if (queue) fill_words(ctx, queue, qwords, 0);
@@ -1567,7 +1662,23 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
     for (auto& st : steps) {
       const int K = int(st.jobs.size());
       const int64_t* dbase = reinterpret_cast<const int64_t*>(dblob + st.t2);
-      if (st.kind == kStepDilate) {
+      if (st.kind == kStepDilate && direct) {
+        // (every tile writes its columns' lengths, also one that gives up)
+        fill_words(ctx, len + st.C, 2, 0);
+        if (st.sum_base[K] > 0) {
+          hipLaunchKernelGGL(vo::summary_batch_kernel<T>, dim3(unsigned(st.sum_base[K])), dim3(vo::kWave * vo::kSide), 0,
+                             ctx->stream, reinterpret_cast<const vo::SummaryArgs<T>*>(dblob + st.t0),
+                             reinterpret_cast<const int64_t*>(dblob + st.t4), K);
+          check(ctx, hipGetLastError(), "batched pass1 launch");
+        }
+        for (int c = 0; c < 3; ++c)
+          if (st.cls_t1[c] > st.cls_t0[c])
+            launch_direct_batch<T>(ctx, c, st.cls_rmax[c], reinterpret_cast<const vo::DirectArgs<T>*>(dblob + st.t1), dbase,
+                                   K, st.cls_t0[c], st.cls_t1[c] - st.cls_t0[c]);
+        check(ctx, hipGetLastError(), "batched pass2 launch");
+        ++di;
+        finish_dilation(st);
+      } else if (st.kind == kStepDilate) {
         const auto* d1 = reinterpret_cast<const vo::Pass1ZArgs<T>*>(dblob + st.t0);
         const auto* d2 = reinterpret_cast<const vo::Pass2GArgs<T>*>(dblob + st.t1);
         // columns a failed job never writes keep length 0
@@ -1595,13 +1706,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
         }
         check(ctx, hipGetLastError(), "batched pass2 launch");
         ++di;
-        exclusive_scan(ctx, len, st.off, st.C + 1);
-        if (st.C > 0) {  // (a step over empty grids only has its one offset)
-          hipLaunchKernelGGL(vo::gather_kernel<T>, dim3(blocks_for(st.C, 256)), dim3(256), 0, ctx->stream, st.C,
-                             static_cast<const T*>(o_z), o_start, len, st.off, static_cast<T*>(st.z), INT64_MAX,
-                             INT64_MAX);
-          check(ctx, hipGetLastError(), "gather launch");
-        }
+        finish_dilation(st);
       } else {
         const auto* dt = reinterpret_cast<const vo::ColumnJob<T>*>(dblob + st.t0);
         const dim3 grid(blocks_for(std::max<int64_t>(st.C, 1), 256));

@@ -21,8 +21,12 @@
 namespace vo {
 
 constexpr int kSide = 8;               // an output tile, and a block of source columns, is kSide x kSide
-constexpr int kDirectWaves = 4;        // tiles (wavefronts) per workgroup: they share the H table in LDS
-constexpr int kDirectLdsTableMax = 31; // largest radius whose H table is staged in LDS
+// Largest radius whose H table is staged in LDS (2.3 KB): one wavefront per
+// workgroup lets the tiles of a launch end one by one, and a larger table of
+// its own costs waves.  Against four wavefronts sharing tables up to R = 31:
+// 1024^2 R = 16 402 -> 392 us (FP64 510 -> 404), R = 64 390 -> 354, 1896^2
+// closing at R = 48 1577 -> 1455, 1000^2 at R = 4 1640 -> 1523.
+constexpr int kDirectLdsTableMax = 9;
 constexpr int kDirectMaxR = 255;       // largest radius this form takes
 constexpr int kDirectMaxList = 512;    // longest list it grows to; the sweeps take volumes that need more
 // Sizes that go with the LDS entries of a lane's list: segments and columns
@@ -150,6 +154,18 @@ __global__ __launch_bounds__(kWave* kSide) void summary_kernel(SummaryArgs<T> g)
   __shared__ int s_cnt[kSide * kSide];
   const int ngx = (g.nbx + kSide - 1) / kSide;
   summary_rows(g, int(blockIdx.x) % ngx, int(blockIdx.x) / ngx, s_row, s_cnt);
+}
+
+// Batched: job j owns the workgroups [base[j], base[j + 1]).
+template <class T>
+__global__ __launch_bounds__(kWave* kSide) void summary_batch_kernel(const SummaryArgs<T>* jobs, const int64_t* base,
+                                                                     int njobs) {
+  __shared__ Ends<T> s_row[kSide * kSide];
+  __shared__ int s_cnt[kSide * kSide];
+  const int j = find_job(base, njobs, blockIdx.x);
+  const SummaryArgs<T> g = jobs[j];
+  const int i = int(blockIdx.x - base[j]), ngx = (g.nbx + kSide - 1) / kSide;
+  summary_rows(g, i % ngx, i / ngx, s_row, s_cnt);
 }
 
 template <class T>
@@ -817,26 +833,49 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
 
 extern __shared__ double vo_direct_htab[];
 
-template <class T, int kList, bool kLdsTable, int kSplit>
-__global__ __launch_bounds__(kWave* (kSplit > 1 ? kSplit : kDirectWaves), kSplit > 1 || kList > 4 ? 2 : 4) void direct_kernel(
-    DirectArgs<T> g, int ntiles) {
-  constexpr int kWaves = kSplit > 1 ? kSplit : kDirectWaves;
-  __shared__ DirectSmem<T, kList> sm[kWaves];
-  const double* htab = g.htab;
+// The H table of radius rint, staged in the workgroup's LDS or where it is.
+template <bool kLdsTable>
+__device__ __forceinline__ const double* stage_htab(const double* htab, int rint) {
   if constexpr (kLdsTable) {
-    const int W = direct_htab_width(g.rint);
-    for (int i = threadIdx.x; i < W * W; i += kWave * kWaves) vo_direct_htab[i] = g.htab[i];
+    const int W = direct_htab_width(rint);
+    for (int i = threadIdx.x; i < W * W; i += blockDim.x) vo_direct_htab[i] = htab[i];
     __syncthreads();
-    htab = vo_direct_htab;
+    return vo_direct_htab;
+  } else {
+    return htab;
   }
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int64_t b = xcd_tile(blockIdx.x, gridDim.x), i = kSplit > 1 ? b : b * kDirectWaves + w;
-  if (i >= ntiles) return;  // (a split tile's wavefronts all stay)
+}
+
+// Registers: four waves per SIMD, where the short lists' LDS allows them.
+template <int kList, int kSplit>
+constexpr int direct_waves() {
+  return kSplit > 1 || kList > 4 ? 2 : 4;
+}
+
+// One tile per workgroup of kSplit wavefronts.
+template <class T, int kList, bool kLdsTable, int kSplit>
+__global__ __launch_bounds__(kWave* kSplit, (direct_waves<kList, kSplit>())) void direct_kernel(DirectArgs<T> g) {
+  __shared__ DirectSmem<T, kList> sm[kSplit];
+  const double* htab = stage_htab<kLdsTable>(g.htab, g.rint);
+  const int64_t i = xcd_tile(blockIdx.x, gridDim.x);
   const int tile = g.only ? g.only[i] : int(i);
-  if constexpr (kSplit > 1)
-    direct_tile<T, kList, kSplit>(g, tile, i, sm, w, htab);
-  else
-    direct_tile<T, kList, 1>(g, tile, i, sm + w, 0, htab);
+  const int part = kSplit > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;
+  direct_tile<T, kList, kSplit>(g, tile, i, sm, part, htab);
+}
+
+// Batched: job j owns the global tiles [tile_base[j], tile_base[j + 1]); this
+// launch covers the n tiles from t0 on (one radius class).
+template <class T, int kList, bool kLdsTable>
+__global__ __launch_bounds__(kWave, (direct_waves<kList, 1>())) void direct_batch_kernel(const DirectArgs<T>* jobs,
+                                                                                    const int64_t* tile_base, int njobs,
+                                                                                    int64_t t0, int64_t n) {
+  __shared__ DirectSmem<T, kList> sm[1];
+  const int64_t t = t0 + xcd_chunk_tile(blockIdx.x, n);
+  const int j = find_job(tile_base, njobs, t);
+  const DirectArgs<T> g = jobs[j];
+  const double* htab = stage_htab<kLdsTable>(g.htab, g.rint);
+  const int64_t i = t - tile_base[j];
+  direct_tile<T, kList, 1>(g, int(i), i, sm, 0, htab);
 }
 
 }  // namespace vo
