@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "../../include/voroffset_hip.h"
+#include "vo_assemble.hpp"
 #include "vo_direct.hpp"
 #include "vo_parity.hpp"
 #include "vo_raster.hpp"
@@ -60,8 +61,17 @@ struct Tuning {
 // R = 6.4: 400 -> 191 us, 212 x 118 closing at R = 27: 466 -> 171, 64 x 48 at
 // R = 4: 255 -> 228; above, the wavefronts' weaker covers cost more than they
 // give: 216 x 310 at R = 2, 1053 tiles, 340 -> 513).
-constexpr int kDirectSplit = 4, kDirectSplitTiles = 512;
-inline int direct_split(int64_t ntiles) { return ntiles <= kDirectSplitTiles ? kDirectSplit : 1; }
+// Where the volume is known to hold few segments per column there is little
+// cover to lose, and two wavefronts a tile shorten the tail of up to 6144
+// tiles: the closing of 544^2 tubes at R = 5 957 -> 728 us in its last
+// dilation, of 336^2 at R = 3 293 -> 216, 628^2 tubes at R = 8 303 -> 276 (dense
+// columns: 839 x 339 at R = 4.8 382 -> 508).
+constexpr int kDirectSplitTiles = 512, kDirectSplitSparseTiles = 6144;
+constexpr int64_t kDirectSparse = 6;  // endpoints per column
+inline int direct_split(int64_t ntiles, int64_t ncols, int64_t endpoints) {
+  if (ntiles <= kDirectSplitTiles) return 4;
+  return ntiles <= kDirectSplitSparseTiles && endpoints >= 0 && endpoints <= kDirectSparse * ncols ? 2 : 1;
+}
 // Entries of a lane's interval list kept in LDS: the long list where columns
 // keep several intervals (small radii) or LDS does not decide how many waves
 // fit (split tiles), the short one elsewhere.
@@ -125,6 +135,7 @@ enum Slot {
   kM_SLO, kM_SHI, kM_CHI,                                    // pass-1 block and column summaries
   kX_SCR, kX_N1, kX_N2, kX_LEN, kX_OFF, kX_Z, kX_LENGTH, kX_SEGS, kX_SUM,  // parity metrics
   kV_WORD, kV_TAB, kV_BASE,                // device-side input check
+  kA_STATE,  // what the chained scan keeps
   kD_COL, kD_AT, kD_BLK, kD_BCNT, kD_TAB,  // one-pass dilation: summaries, H table and block order
   kB_OUT,                                  // + (stage * 3 + kind) * 2 (+1 for z): stage outputs
   kSLOTS = kB_OUT + 4 * 3 * 2
@@ -134,7 +145,9 @@ struct DevVol {
   int nx = 0, ny = 0;
   const int64_t* off = nullptr;
   const void* z = nullptr;
-  int64_t count = 0;
+  int64_t count = 0;     // endpoints (-1: not known on the host)
+  int64_t est = -1;      // at least its endpoints, where the host knows a bound (-1: none)
+  bool pending = false;  // the count is in host_words[4] after the next synchronisation
 };
 
 }  // namespace
@@ -210,6 +223,7 @@ struct vo_context {
   int dtab_norder = 0;
   bool two_pass = false;  // VO_PASS1=zsweep, vo_pass1, vo_autotune: keep to the two sweeps
   int direct_cap = 24;    // intervals per list of the one-pass form (grows on overflow)
+  bool chain_dirty = false;  // a call failed: the chained scan's words may not be zero
   int64_t spec_out = 0;  // endpoints the next dilation's output is first sized for
   // an input check left to the pass 1 of the operation's first dilation
   // (word == null: none pending); see defer_input_check
@@ -335,6 +349,21 @@ void exclusive_scan(vo_context* ctx, const int64_t* len, int64_t* off, int64_t n
   check(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, len, off, int(n), ctx->stream), "scan size");
   void* t = ws(ctx, kSCAN_TMP, tmp);
   check(ctx, hipcub::DeviceScan::ExclusiveSum(t, tmp, len, off, int(n), ctx->stream), "scan");
+}
+
+unsigned assemble_blocks(int64_t n) { return blocks_for(n, vo::kAssembleThreads * vo::assemble_items(n)); }
+
+// The chained scan's words for n columns, zero (the kernels leave them so; a
+// call that failed may not have).
+vo::AssembleState assemble_state(vo_context* ctx, int64_t n) {
+  const size_t need = 64 + size_t(assemble_blocks(n)) * sizeof(unsigned long long);
+  const size_t had = ctx->buf[kA_STATE].bytes;
+  char* p = static_cast<char*>(ws(ctx, kA_STATE, need));
+  if (ctx->buf[kA_STATE].bytes != had || ctx->chain_dirty) {
+    check(ctx, hipMemsetAsync(p, 0, ctx->buf[kA_STATE].bytes, ctx->stream), "memset");
+    ctx->chain_dirty = false;
+  }
+  return vo::AssembleState{reinterpret_cast<unsigned*>(p), reinterpret_cast<unsigned long long*>(p + 64)};
 }
 
 int64_t read_word(vo_context* ctx, const int64_t* dptr) {
@@ -556,10 +585,14 @@ void launch_direct(vo_context* ctx, int rint, int split, const vo::DirectArgs<T>
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(unsigned(ntiles)), dim3(vo::kWave * split), lds, ctx->stream, a);
   };
-  if (split > 1 && lds_table)
-    launch(vo::direct_kernel<T, kDirectListLong, true, kDirectSplit>);
-  else if (split > 1)
-    launch(vo::direct_kernel<T, kDirectListLong, false, kDirectSplit>);
+  if (split == 4 && lds_table)
+    launch(vo::direct_kernel<T, kDirectListLong, true, 4>);
+  else if (split == 4)
+    launch(vo::direct_kernel<T, kDirectListLong, false, 4>);
+  else if (split == 2 && lds_table)
+    launch(vo::direct_kernel<T, kDirectListLong, true, 2>);
+  else if (split == 2)
+    launch(vo::direct_kernel<T, kDirectListLong, false, 2>);
   else if (rint <= kDirectSmallR)
     launch(vo::direct_kernel<T, kDirectListLong, true, 1>);
   else if (lds_table)
@@ -605,7 +638,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   int64_t* o_start = static_cast<int64_t*>(slot_ptr(ctx, kO_START));
   int64_t* o_len = static_cast<int64_t*>(slot_ptr(ctx, kO_LEN));
   int cap = ctx->direct_cap;
-  const int split = direct_split(ntiles), in_lds = direct_list(rint, split);
+  const int split = direct_split(ntiles, ncols, in.count >= 0 ? in.count : in.est), in_lds = direct_list(rint, split);
   const int W = vo::direct_htab_width(rint);
   DirectTable tab;  // outlives its upload (a synchronisation follows)
   const bool cached = !ctx->arena.on && ctx->dtab_R == R && ctx->dtab_axis == int(along_x) && ctx->dtab_at;
@@ -688,19 +721,25 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
     launch_direct<T>(ctx, rint, split, a, int(todo));
     check(ctx, hipGetLastError(), "pass2 gather launch");
     check(ctx, hipEventRecord(ctx->ev[2], ctx->stream), "event");
-    exclusive_scan(ctx, o_len, out_off, ncols + 1);
-    hipLaunchKernelGGL(vo::report_words_kernel, dim3(1), dim3(1), 0, ctx->stream, out_off + ncols, status, a.tile_list,
-                       chk_word, ctx->host_words);
-    check(ctx, hipGetLastError(), "report words");
-    // the CSR copy before the synchronisation, into an output sized like the
-    // last result plus a quarter (see dilate)
     int64_t spec = 0;
-    if (!ctx->arena.on) {
+    if (ctx->arena.on) {
+      exclusive_scan(ctx, o_len, out_off, ncols + 1);
+      hipLaunchKernelGGL(vo::report_words_kernel, dim3(1), dim3(1), 0, ctx->stream, out_off + ncols, status, a.tile_list,
+                         chk_word, ctx->host_words);
+      check(ctx, hipGetLastError(), "report words");
+    } else {
+      // offsets, CSR and report in one launch before the synchronisation, the
+      // CSR into an output sized like the last result plus a quarter (columns
+      // that would not fit are skipped and copied afterwards)
       spec = std::max<int64_t>(ctx->spec_out, 16);
       T* oz = static_cast<T*>(ws(ctx, out_z_slot, size_t(spec) * sizeof(T)));
-      hipLaunchKernelGGL(vo::gather_kernel<T>, dim3(blocks_for(ncols, 256)), dim3(256), 0, ctx->stream, ncols,
-                         static_cast<const T*>(o_z), o_start, o_len, out_off, oz, INT64_MAX, spec);
-      check(ctx, hipGetLastError(), "gather launch");
+      const vo::AssembleState st = assemble_state(ctx, ncols);
+      auto* k = vo::assemble_items(ncols) == 1 ? vo::assemble_dilation_kernel<T, 1>
+                                               : vo::assemble_dilation_kernel<T, vo::kAssembleMany>;
+      hipLaunchKernelGGL(k, dim3(assemble_blocks(ncols)), dim3(vo::kAssembleThreads), 0, ctx->stream, ncols,
+                         static_cast<const T*>(o_z), o_start, o_len, out_off, oz, spec, st,
+                         vo::AssembleReport{ctx->host_words, status, a.tile_list, chk_word});
+      check(ctx, hipGetLastError(), "assemble launch");
     }
     sync(ctx);
     const int64_t nfall = int64_t(uint32_t(ctx->host_words[2]));
@@ -1138,6 +1177,37 @@ template <class T>
 DevVol column_transform(vo_context* ctx, bool ring, const DevVol& in, T lo, T hi, int off_slot, int z_slot) {
   const int onx = ring ? in.nx + 2 : in.nx - 2, ony = ring ? in.ny + 2 : in.ny - 2;
   const int64_t n = int64_t(onx) * ony;
+  if (!ctx->arena.on && n > 0) {
+    // A complement adds at most two endpoints to a column, so with the input's
+    // count there is room for the result before its size is known, and
+    // lengths, offsets and data are one launch with nothing to wait for.
+    const int64_t in_cols = int64_t(in.nx) * in.ny;
+    // (a volume the caller keeps on the device: its last offset, which is no
+    // less than what its columns hold)
+    const int64_t count = in.count >= 0 ? in.count : (in_cols ? read_word(ctx, in.off + in_cols) : 0);
+    const int64_t cap = count + 2 * n;
+    int64_t* off = static_cast<int64_t*>(ws(ctx, off_slot, (n + 1) * sizeof(int64_t)));
+    T* z = static_cast<T*>(ws(ctx, z_slot, size_t(std::max<int64_t>(cap, 1)) * sizeof(T)));
+    const vo::ColumnJob<T> job{ring ? in.nx : onx, ring ? in.ny : ony, in.off, static_cast<const T*>(in.z), lo, hi, nullptr,
+                               nullptr, z};
+    const vo::AssembleState st = assemble_state(ctx, n);
+    vo::AssembleReport rep;
+    if (!ring) rep.host = ctx->host_words + 4;  // the result's size, for whoever synchronises next
+    const bool one = vo::assemble_items(n) == 1;
+    auto* k = ring ? (one ? vo::assemble_complement_kernel<T, true, 1> : vo::assemble_complement_kernel<T, true, vo::kAssembleMany>)
+                   : (one ? vo::assemble_complement_kernel<T, false, 1> : vo::assemble_complement_kernel<T, false, vo::kAssembleMany>);
+    hipLaunchKernelGGL(k, dim3(assemble_blocks(n)), dim3(vo::kAssembleThreads), 0, ctx->stream, job, n, off, cap, st, rep);
+    check(ctx, hipGetLastError(), "complement launch");
+    DevVol out;
+    out.nx = onx;
+    out.ny = ony;
+    out.off = off;
+    out.z = z;
+    out.count = -1;
+    out.est = cap;
+    out.pending = !ring;
+    return out;
+  }
   int64_t* len = static_cast<int64_t*>(ws(ctx, kO_LEN, (n + 1) * sizeof(int64_t)));
   int64_t* off = static_cast<int64_t*>(ws(ctx, off_slot, (n + 1) * sizeof(int64_t)));
   auto launch = [&](int phase, const int64_t* o, T* z) {
@@ -1351,6 +1421,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
     vol[j].ny = jb.in.ny;
     vol[j].off = jb.in.offsets;
     vol[j].z = jb.in.z;
+    vol[j].count = -1;
   }
   if (t1) *t1 = 0;
   if (t2) *t2 = 0;
@@ -1983,6 +2054,7 @@ void autotune(vo_context* ctx, const vo_volume* sample, int n, const double* rad
   in.ny = sample->ny;
   in.off = sample->offsets;
   in.z = sample->z;
+  in.count = -1;
   const int forced = ctx->zsweep_events;
   struct Sweeps {  // the shapes it tunes are the two sweeps'
     vo_context* c;
@@ -2051,10 +2123,12 @@ int guarded(vo_context* ctx, const std::function<void()>& body) {
   } catch (const Failure& f) {
     ctx->check_input = false;
     ctx->fused.word = nullptr;
+    ctx->chain_dirty = true;
     return f.code;
   } catch (const std::exception& e) {
     ctx->check_input = false;
     ctx->fused.word = nullptr;
+    ctx->chain_dirty = true;
     ctx->error = e.what();
     return VO_ERR_ARGUMENT;
   }
@@ -2268,6 +2342,10 @@ void morph_host(vo_context* ctx, int op, double R, const vo_volume* in, vo_resul
   DevVol v = upload_host<T>(ctx, in, shift);
   DevVol r = v;
   if (op != VO_OP_NOOP) r = run_op<T>(ctx, op, v, R, in->z_lo - shift, in->z_hi - shift, t1, t2);
+  if (r.pending) {
+    sync(ctx);
+    r.count = ctx->host_words[4];
+  }
   auto* res = new vo_result;
   res->nx = r.nx;
   res->ny = r.ny;
@@ -2586,6 +2664,7 @@ int vo_morph_device(vo_context* ctx, int op, int precision, double radius, const
     v.ny = in->ny;
     v.off = in->offsets;
     v.z = in->z;
+    v.count = -1;
     DevVol r = v;
     if (op == VO_OP_NOOP) {
       const int64_t n = int64_t(in->nx) * in->ny;
@@ -2602,6 +2681,7 @@ int vo_morph_device(vo_context* ctx, int op, int precision, double radius, const
       fail(ctx, VO_ERR_ARGUMENT, "unknown precision");
     }
     sync(ctx);
+    if (r.pending) r.count = ctx->host_words[4];
     out->nx = r.nx;
     out->ny = r.ny;
     out->offsets = r.off;

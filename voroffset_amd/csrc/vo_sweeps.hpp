@@ -972,15 +972,13 @@ struct ColumnJob {  // one volume of a column-parallel kernel
   T* out;
 };
 
+// The column's length in endpoints; its data too where `out` is given.
 template <class T>
-__device__ void ring_column(const ColumnJob<T>& g, int64_t C, int phase) {
+__device__ int64_t ring_column(const ColumnJob<T>& g, int64_t C, T* out) {
   const int nx = g.nx, ny = g.ny;
   const int64_t* off = g.off;
   const T* z = g.z;
   const T lo = g.lo, hi = g.hi;
-  int64_t* out_len = g.out_len;
-  const int64_t* out_off = g.out_off;
-  T* out = g.out;
   const int NX = nx + 2;
   const int X = int(C % NX), Y = int(C / NX);
   int64_t s = 0, n = 0;
@@ -990,77 +988,79 @@ __device__ void ring_column(const ColumnJob<T>& g, int64_t C, int phase) {
     n = off[c + 1] - s;
   }
   if (n == 0) {
-    if (phase == 0) {
-      out_len[C] = 2;
-    } else {
-      out[out_off[C]] = lo;
-      out[out_off[C] + 1] = hi;
+    if (out) {
+      out[0] = lo;
+      out[1] = hi;
     }
-    return;
+    return 2;
   }
   const bool drop_first = z[s] == lo, drop_last = z[s + n - 1] == hi;
-  if (phase == 0) {
-    out_len[C] = n + (drop_first ? -1 : 1) + (drop_last ? -1 : 1);
-    return;
+  if (out) {
+    int64_t w = 0;
+    if (!drop_first) out[w++] = lo;
+    for (int64_t i = drop_first ? 1 : 0; i < (drop_last ? n - 1 : n); ++i) out[w++] = z[s + i];
+    if (!drop_last) out[w++] = hi;
   }
-  int64_t w = out_off[C];
-  if (!drop_first) out[w++] = lo;
-  for (int64_t i = drop_first ? 1 : 0; i < (drop_last ? n - 1 : n); ++i) out[w++] = z[s + i];
-  if (!drop_last) out[w++] = hi;
-}
-
-template <class T>
-__global__ void ring_complement_kernel(ColumnJob<T> g, int phase) {
-  const int64_t C = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (C >= int64_t(g.nx + 2) * (g.ny + 2)) return;
-  ring_column(g, C, phase);
+  return n + (drop_first ? -1 : 1) + (drop_last ? -1 : 1);
 }
 
 // Crop the ring and complement within [lo, hi] with parity counting
 // (negateInv, Voronoi.cpp:57-89; negate_ray_range, MorphologyOperators.cpp:282-315).
 // (here nx, ny are the output grid: the input is (nx + 2) x (ny + 2))
 template <class T>
-__device__ void crop_column(const ColumnJob<T>& g, int64_t c, int phase) {
+__device__ int64_t crop_column(const ColumnJob<T>& g, int64_t c, T* out) {
   const int nx = g.nx;
   const int64_t* off = g.off;
   const T* z = g.z;
   const T lo = g.lo, hi = g.hi;
-  int64_t* out_len = g.out_len;
-  const int64_t* out_off = g.out_off;
-  T* out = g.out;
   const int x = int(c % nx), y = int(c / nx);
   const int64_t C = int64_t(x + 1) + int64_t(nx + 2) * (y + 1);
   const int64_t s = off[C], n = off[C + 1] - s;
   if (n == 0) {
-    if (phase == 0) {
-      out_len[c] = 2;
-    } else {
-      out[out_off[c]] = lo;
-      out[out_off[c] + 1] = hi;
+    if (out) {
+      out[0] = lo;
+      out[1] = hi;
     }
-    return;
+    return 2;
   }
   int64_t head = 0;
   while (head < n && z[s + head] <= lo) ++head;
   int64_t tail = 0;
   while (tail < n - head && z[s + n - 1 - tail] >= hi) ++tail;
   const bool add_lo = head % 2 == 0, add_hi = tail % 2 == 0;
-  const int64_t mid = n - head - tail;
-  if (phase == 0) {
-    out_len[c] = mid + (add_lo ? 1 : 0) + (add_hi ? 1 : 0);
-    return;
+  if (out) {
+    int64_t w = 0;
+    if (add_lo) out[w++] = lo;
+    for (int64_t i = head; i < n - tail; ++i) out[w++] = z[s + i];
+    if (add_hi) out[w++] = hi;
   }
-  int64_t w = out_off[c];
-  if (add_lo) out[w++] = lo;
-  for (int64_t i = head; i < n - tail; ++i) out[w++] = z[s + i];
-  if (add_hi) out[w++] = hi;
+  return n - head - tail + (add_lo ? 1 : 0) + (add_hi ? 1 : 0);
+}
+template <class T, bool kRing>
+__device__ int64_t complement_column(const ColumnJob<T>& g, int64_t c, T* out) {
+  return kRing ? ring_column(g, c, out) : crop_column(g, c, out);
+}
+// Phase 0 writes the column's length, phase 1 its data.
+template <class T, bool kRing>
+__device__ void complement_phase(const ColumnJob<T>& g, int64_t c, int phase) {
+  if (phase == 0)
+    g.out_len[c] = complement_column<T, kRing>(g, c, nullptr);
+  else
+    complement_column<T, kRing>(g, c, g.out + g.out_off[c]);
+}
+
+template <class T>
+__global__ void ring_complement_kernel(ColumnJob<T> g, int phase) {
+  const int64_t C = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (C >= int64_t(g.nx + 2) * (g.ny + 2)) return;
+  complement_phase<T, true>(g, C, phase);
 }
 
 template <class T>
 __global__ void crop_complement_kernel(ColumnJob<T> g, int phase) {
   const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (c >= int64_t(g.nx) * g.ny) return;
-  crop_column(g, c, phase);
+  complement_phase<T, false>(g, c, phase);
 }
 
 // Batched forms: job j owns output columns [col_base[j], col_base[j + 1]).
@@ -1070,7 +1070,7 @@ __global__ void ring_complement_batch_kernel(const ColumnJob<T>* jobs, const int
   const int64_t C = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (C >= col_base[njobs]) return;
   const int j = find_job(col_base, njobs, C);
-  ring_column(jobs[j], C - col_base[j], phase);
+  complement_phase<T, true>(jobs[j], C - col_base[j], phase);
 }
 
 template <class T>
@@ -1079,7 +1079,7 @@ __global__ void crop_complement_batch_kernel(const ColumnJob<T>* jobs, const int
   const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (c >= col_base[njobs]) return;
   const int j = find_job(col_base, njobs, c);
-  crop_column(jobs[j], c - col_base[j], phase);
+  complement_phase<T, false>(jobs[j], c - col_base[j], phase);
 }
 
 // Final offsets of a batch: job j's offsets off_j[0 .. ncols_j] (absolute
