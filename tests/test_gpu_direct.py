@@ -8,6 +8,7 @@ import os
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from voroffset_amd import _native, synth
@@ -118,3 +119,46 @@ def test_points_and_touching_segments(contexts, prec):
     vol = column_volume(23, 17, cols, 40.0)
     for r in (1.0, 2.5, 5.0, 13.0):
         both(contexts, vol, "dilation", prec, r)
+
+
+def on_device(ctx, vol, op, prec, r):
+    """The call on a volume whose size only the device knows."""
+    t = torch.float32 if prec == "fp32" else torch.float64
+    off, z = torch.from_numpy(vol.off).cuda(), torch.from_numpy(vol.z).to(t).cuda()
+    if z.numel() == 0:
+        z = torch.zeros(1, dtype=t, device="cuda")
+    torch.cuda.synchronize()
+    out, count, _ = ctx.morph_device(op, prec, r, vol.nx, vol.ny, off.data_ptr(), z.data_ptr(), *vol.z_range())
+    got_off = torch.zeros(out.nx * out.ny + 1, dtype=torch.int64, device="cuda")
+    got = torch.zeros(max(count, 1), dtype=t, device="cuda")
+    copies = [(got_off.data_ptr(), out.offsets, got_off.numel() * 8)]
+    if count:
+        copies.append((got.data_ptr(), out.z, count * got.element_size()))
+    torch.cuda.synchronize()
+    ctx.copy_device(copies)
+    return got_off.cpu().numpy(), got[:count].cpu().numpy()
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("lam", [1.0, 4.0])
+@pytest.mark.parametrize("op,r", [("dilation", 2.5), ("dilation", 9.9), ("dilation", 15.5), ("dilation", 16.0),
+                                  ("closing", 2.5), ("closing", 10.0), ("erosion", 3.5), ("opening", 3.0)])
+def test_shared_tiles_of_sparse_volumes(contexts, prec, lam, op, r):
+    """More than 512 tiles, few and many segments a column: known to the host
+    (from host memory) or only to the device, and in a complement."""
+    vol = synth.poisson_columns(233, 150, lam=lam, mean_len=60.0, zmax=600, seed=int(10 * r), z_margin=int(r) + 3)
+    both(contexts, vol, op, prec, r)
+    one, two = [on_device(c, vol, op, prec, r) for c in contexts]
+    assert np.array_equal(one[0], two[0]) and np.array_equal(one[1], two[1])
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 511), (512, 1), (19, 27), (512, 256), (131073, 1), (683, 769)])
+@pytest.mark.parametrize("op", ["dilation", "erosion"])
+def test_offsets_of_one_launch(contexts, nx, ny, op):
+    """Grids at the edges of a workgroup's columns (512 or 2048) and of the
+    rule between the two; small and large results in turn, so that the output
+    is once too small for the launch; empty columns and an empty result."""
+    for lam in (0.0, 3.0, 0.2, 6.0):
+        vol = synth.poisson_columns(nx, ny, lam=lam, zmax=200, mean_len=30.0, seed=3, z_margin=8)
+        one, two = [on_device(c, vol, op, "fp32", 1.5) for c in contexts]
+        assert np.array_equal(one[0], two[0]) and np.array_equal(one[1], two[1])

@@ -61,16 +61,24 @@ struct Tuning {
 // R = 6.4: 400 -> 191 us, 212 x 118 closing at R = 27: 466 -> 171, 64 x 48 at
 // R = 4: 255 -> 228; above, the wavefronts' weaker covers cost more than they
 // give: 216 x 310 at R = 2, 1053 tiles, 340 -> 513).
-// Where the volume is known to hold few segments per column there is little
-// cover to lose, and two wavefronts a tile shorten the tail of up to 6144
-// tiles: the closing of 544^2 tubes at R = 5 957 -> 728 us in its last
-// dilation, of 336^2 at R = 3 293 -> 216, 628^2 tubes at R = 8 303 -> 276 (dense
-// columns: 839 x 339 at R = 4.8 382 -> 508).
+// Where the volume holds few segments per column (the host knows, or the
+// kernels look: see direct_kernel) there is little cover to lose, and at radii
+// below 16 two wavefronts a tile shorten the tail of up to 6144 tiles: 544^2
+// tubes at R = 10 687 -> 623 us, 336^2 tubes closed at R = 3 291 -> 214 in the last
+// dilation, 512^2 solids at R = 4 295 -> 280.  Denser columns lose (1531 x 219 at
+// R = 7.3, 5 endpoints a column, 234 -> 316; 839 x 339 at R = 4.8, 6.4 of them,
+// 360 -> 503), and so do large radii (1097 x 310 solids at R = 35 698 -> 758).  A
+// complement's columns have two endpoints more, and what the dilation before
+// it parted: four more are allowed (the last dilation of 544^2 tubes closed
+// at R = 5 910 -> 720; the other side is an erosion of 1531 x 219 short random
+// segments, 78 -> 131).
 constexpr int kDirectSplitTiles = 512, kDirectSplitSparseTiles = 6144;
-constexpr int64_t kDirectSparse = 6;  // endpoints per column
-inline int direct_split(int64_t ntiles, int64_t ncols, int64_t endpoints) {
+constexpr int64_t kDirectSparse = 4;  // endpoints per column
+constexpr int kDirectSparseR = 16;
+constexpr int64_t direct_sparse(int64_t ncols, bool outer) { return (kDirectSparse + 4 * outer) * ncols; }
+inline int direct_split(int64_t ntiles, int64_t endpoints, int64_t sparse, int rint) {
   if (ntiles <= kDirectSplitTiles) return 4;
-  return ntiles <= kDirectSplitSparseTiles && endpoints >= 0 && endpoints <= kDirectSparse * ncols ? 2 : 1;
+  return ntiles <= kDirectSplitSparseTiles && rint < kDirectSparseR && endpoints >= 0 && endpoints <= sparse ? 2 : 1;
 }
 // Entries of a lane's interval list kept in LDS: the long list where columns
 // keep several intervals (small radii) or LDS does not decide how many waves
@@ -146,7 +154,7 @@ struct DevVol {
   const int64_t* off = nullptr;
   const void* z = nullptr;
   int64_t count = 0;     // endpoints (-1: not known on the host)
-  int64_t est = -1;      // at least its endpoints, where the host knows a bound (-1: none)
+  bool outer = false;    // columns end in two endpoints that a ring complement added
   bool pending = false;  // the count is in host_words[4] after the next synchronisation
 };
 
@@ -638,7 +646,10 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   int64_t* o_start = static_cast<int64_t*>(slot_ptr(ctx, kO_START));
   int64_t* o_len = static_cast<int64_t*>(slot_ptr(ctx, kO_LEN));
   int cap = ctx->direct_cap;
-  const int split = direct_split(ntiles, ncols, in.count >= 0 ? in.count : in.est), in_lds = direct_list(rint, split);
+  const int64_t sparse = direct_sparse(ncols, in.outer);
+  const int split = direct_split(ntiles, in.count, sparse, rint), in_lds = direct_list(rint, split);
+  // (the split a sparse volume would take, where only the device knows)
+  const int sparse_split = in.count >= 0 || ctx->arena.on ? split : direct_split(ntiles, 0, sparse, rint);
   const int W = vo::direct_htab_width(rint);
   DirectTable tab;  // outlives its upload (a synchronisation follows)
   const bool cached = !ctx->arena.on && ctx->dtab_R == R && ctx->dtab_axis == int(along_x) && ctx->dtab_at;
@@ -646,7 +657,10 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   const size_t hbytes = size_t(W) * W * sizeof(double);
   int norder = cached ? ctx->dtab_norder : int(tab.order.size());
   const size_t tbytes = hbytes + size_t(norder) * sizeof(int2);
-  auto list_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * split * 2 * (c - in_lds) * vo::kWave * sizeof(double); };
+  auto list_bytes = [&](int64_t tiles, int c) {
+    const int sparse_lds = direct_list(rint, sparse_split);
+    return size_t(tiles) * std::max(split * (c - in_lds), sparse_split * (c - sparse_lds)) * 2 * vo::kWave * sizeof(double);
+  };
   auto out_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * 2 * c * vo::kWave * sizeof(T); };
   vo::Ends<T>*col, *blk;
   uint64_t* at;
@@ -718,6 +732,14 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   int64_t total = -1;
   bool copied = false;
   for (;;) {
+    if (sparse_split != split) {
+      a.least = INT64_MIN;
+      a.most = sparse;
+      launch_direct<T>(ctx, rint, sparse_split, a, int(todo));
+      check(ctx, hipGetLastError(), "pass2 gather launch");
+      a.least = a.most + 1;
+      a.most = INT64_MAX;
+    }
     launch_direct<T>(ctx, rint, split, a, int(todo));
     check(ctx, hipGetLastError(), "pass2 gather launch");
     check(ctx, hipEventRecord(ctx->ev[2], ctx->stream), "event");
@@ -729,9 +751,10 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
       check(ctx, hipGetLastError(), "report words");
     } else {
       // offsets, CSR and report in one launch before the synchronisation, the
-      // CSR into an output sized like the last result plus a quarter (columns
-      // that would not fit are skipped and copied afterwards)
-      spec = std::max<int64_t>(ctx->spec_out, 16);
+      // CSR into an output sized like the last result plus a quarter or what
+      // the buffer has room for (a closing's two results differ; columns that
+      // would not fit are skipped and copied afterwards)
+      spec = std::max<int64_t>(std::max<int64_t>(ctx->spec_out, 16), int64_t(ctx->buf[out_z_slot].bytes / sizeof(T)));
       T* oz = static_cast<T*>(ws(ctx, out_z_slot, size_t(spec) * sizeof(T)));
       const vo::AssembleState st = assemble_state(ctx, ncols);
       auto* k = vo::assemble_items(ncols) == 1 ? vo::assemble_dilation_kernel<T, 1>
@@ -1204,7 +1227,7 @@ DevVol column_transform(vo_context* ctx, bool ring, const DevVol& in, T lo, T hi
     out.off = off;
     out.z = z;
     out.count = -1;
-    out.est = cap;
+    out.outer = ring;
     out.pending = !ring;
     return out;
   }

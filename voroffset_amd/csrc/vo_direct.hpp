@@ -190,6 +190,7 @@ struct DirectArgs {
   int* tile_list;        // [0] = count, then the tiles whose lists overflowed (null: raise the status)
   int* status;
   const int* only;       // tiles to do (null: all)
+  int64_t least = INT64_MIN, most = INT64_MAX;  // endpoints in the volume for which this launch works
 };
 
 // Lane values combined over the wavefront (result in every lane, scalar).
@@ -852,10 +853,15 @@ constexpr int direct_waves() {
   return kSplit > 1 || kList > 4 ? 2 : 4;
 }
 
-// One tile per workgroup of kSplit wavefronts.
+// One tile per workgroup of kSplit wavefronts.  Where only the device knows
+// how many endpoints the volume has, two launches of different splits go out
+// and the one whose range does not hold them returns at once (its 4,600 empty
+// workgroups cost 3 us at 544^2; reading the count back would cost a wait).
 template <class T, int kList, bool kLdsTable, int kSplit>
 __global__ __launch_bounds__(kWave* kSplit, (direct_waves<kList, kSplit>())) void direct_kernel(DirectArgs<T> g) {
   __shared__ DirectSmem<T, kList> sm[kSplit];
+  const int64_t endpoints = g.off[int64_t(g.nx) * g.ny];
+  if (endpoints < g.least || endpoints > g.most) return;
   const double* htab = stage_htab<kLdsTable>(g.htab, g.rint);
   const int64_t i = xcd_tile(blockIdx.x, gridDim.x);
   const int tile = g.only ? g.only[i] : int(i);
