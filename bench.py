@@ -5,15 +5,15 @@ Workload (one step): dilation by r=16 of a direct dexel volume on a
 1024x1024 grid, z-extent 1024, Poisson(6) segments per column with
 exponential (mean 40 dexel) gaps and lengths, endpoints stored as FP32 on the
 device (predicates and endpoint arithmetic in FP64).  Inputs are resident in
-HBM before the timed region; a step is one vo_morph_device() call (pass 1,
-pass 2, output CSR assembly), synchronised.
+HBM before the timed region; a step is one vo_morph_device() call (block
+summaries, the one-pass dilation, output CSR assembly), synchronised.
 
 Prints ONE JSON line (see the keys below).  `roofline` is computed for the
 dominant kernel from its average duration over the timed steps, measured with
-HIP events that the library records on its own stream around each kernel;
-its byte count is algorithmic: per column pass 1 reads (2*s_in*E + 4) and
-writes (3*m*E + 4), pass 2 reads (3*m*E + 4) and writes (2*s_out*E + 4),
-with E = 4 bytes and m the oracle's pass-1 triple count for this input.
+HIP events that the library records on its own stream around each kernel
+(`pass1_ms` the summaries, `pass2_ms` the one-pass dilation); its byte count
+is algorithmic: per column the input is read once (2*s_in*E + 8) and the
+output written once (2*s_out*E + 8), with E = 4 bytes and 8 of offset.
 `cpu_baseline` times the CPU oracle (the FP64 restatement of `ours`) on a
 bounded crop of the same volume, on this host's cores.
 """
@@ -518,18 +518,13 @@ def main():
     s_in = vol.num_segments() / ncols
     s_out = count / 2 / ncols
     roofline = None
-    if m is not None:
-        b1 = ncols * ((2 * s_in * E + 4) + (3 * m * E + 4))
-        b2 = ncols * ((3 * m * E + 4) + (2 * s_out * E + 4))
-        name, b, ms = ("pass2", b2, p2_ms) if p2_ms >= p1_ms else ("pass1", b1, p1_ms)
+    if R < 256 and not os.environ.get("VO_PASS1"):  # the one-pass form: summaries, then the dilation
+        b = ncols * ((2 * s_in * E + 8) + (2 * s_out * E + 8))
+        name, ms = "direct", p2_ms
         achieved = b / (ms * 1e-3) / 1e9
-        # the instantiation the timed steps ran (FP32 storage, this radius and
-        # slab capacity); counters measured on another one are not attached
-        events = (tuned or {}).get("events_per_slab", 768)
-        nb = {512: 256, 768: 512, 1024: 512, 1536: 512}.get(events, 512)
-        nw = 1 if int(R) <= 31 else (2 if int(R) <= 63 else 4)
-        inst = (f"pass1_zsweep_kernel<float, {events}, {nb}, 320, {nw}>" if name == "pass1"
-                else f"pass2_gather_kernel<float, {'true' if int(R) <= 31 else 'false'}>")
+        # the instantiation the timed steps ran (FP32 storage, this radius);
+        # counters measured on another one are not attached
+        inst = f"direct_kernel<float, {8 if int(R) <= 3 else 3}, {'true' if int(R) <= 9 else 'false'}, 1>"
         traffic, tnote = None, "no counter profile of this kernel in profiles/"
         tpath = os.path.join(ROOT, "profiles", f"traffic_{name}_1024_r16.json")
         if os.path.exists(tpath):
@@ -541,7 +536,7 @@ def main():
         roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic, "traffic_source": tnote,
                     "kernel": inst, "kernel_ms": round(ms, 4), "algorithmic_bytes": int(b),
-                    "step_algorithmic_GBs": round((b1 + b2) / step_s / 1e9, 2)}
+                    "step_algorithmic_GBs": round(b / step_s / 1e9, 2)}
 
     out = {
         "metric": METRIC,

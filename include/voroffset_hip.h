@@ -12,7 +12,8 @@
  * pair: `offsets` (nx*ny + 1 int64) and `z` (float or double endpoints).
  *
  * Conventions (mirroring the reference):
- *   - radius is in dexels; time_1 / time_2 report pass 1 / pass 2 in ms;
+ *   - radius is in dexels; time_1 / time_2 report pass 1 / pass 2 in ms (in
+ *     the one-pass form, radii below 256: its block summaries / the dilation);
  *   - erosion complements on a grid grown by one ring of full columns over
  *     [z_lo - 1, z_hi + 1], dilates, crops and complements within [z_lo, z_hi],
  *     where z_lo = origin_z / spacing and z_hi = z_lo + 2*padding + extent_z / spacing;
@@ -190,7 +191,9 @@ void vo_mesh_free(vo_mesh_result* r);
  * list capacity (8, 16, 24, 32) on `sample` (a device volume of the given
  * precision), `reps` runs each, and keeps the fastest per radius bucket
  * ([0,8), [8,16), [16,32), [32,64), [64,128)) in `ctx`; results do not
- * depend on the choice.  The table can be saved, loaded and read back. */
+ * depend on the choice.  It times and tunes the two-sweep form; a dilation in
+ * one pass (radii below 256, unless VO_PASS1 names a form) has nothing to
+ * tune.  The table can be saved, loaded and read back. */
 int vo_autotune(vo_context* ctx, int precision, const vo_volume* sample, int num_radii, const double* radii,
                 int reps);
 int vo_tuning_save(const vo_context* ctx, const char* path);

@@ -2,6 +2,11 @@
 //
 // Orchestration of one dilation (VoronoiMorphoVorPower::dilation,
 // src/vor3d/VoronoiVorPower.cpp:24-96) on the device:
+//   summary kernel -> the ends and counts of every column and 8 x 8 block
+//   direct kernel  -> per-column output intervals, in one pass over the input
+//   assemble       -> offsets, CSR result and report in one chained scan
+// Radii of 256 and more, lists past the direct form's room, and the forms
+// VO_PASS1 / VO_PASS2 name take two sweeps instead:
 //   pass 1 kernel  -> per-column triples (lo, hi, dy) in a chunked arena
 //   pass 2 kernel  -> per-column output intervals in a chunked arena
 //   exclusive scan of the output lengths + gather -> CSR result

@@ -94,7 +94,8 @@ def footprint_bytes(ncols, endpoints, op, storage_bytes=4, caps=96, ocap=24):
     output arena (2 * ocap endpoints), the start, length and offset words;
     plus the outputs of the job's stages at their bounds (the batch program
     sizes them before it runs).  ocap is the largest list capacity a batch uses (24 when
-    it holds a radius below 6, 16 otherwise)."""
+    it holds a radius below 6, 16 otherwise).  An upper bound: jobs with radii
+    below 256 run in one pass and keep no pass-1 slots."""
     if op not in _DILATIONS:
         raise ValueError(f"unknown operation {op!r}")
     if _DILATIONS[op] == 0:
