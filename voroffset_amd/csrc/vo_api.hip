@@ -140,7 +140,7 @@ enum Slot {
   kSTATUS, kSCAN_TMP, kTILES,
   kV0_OFF, kV0_Z, kV1_OFF, kV1_Z, kV2_OFF, kV2_Z, kV3_OFF, kV3_Z,  // device volumes
   kIN_OFF, kIN_Z,                                                   // staged host input
-  kR_V, kR_F, kR_TCNT, kR_TOFF, kR_TCUR, kR_TTRIS, kR_LEN, kR_OFF, kR_Z,  // rasterizer
+  kR_V, kR_F, kR_TCNT, kR_TOFF, kR_TCUR, kR_TTRIS, kR_LEN, kR_OFF, kR_Z, kR_KEEP,  // rasterizer
   kB_TAB0, kB_TAB1, kB_TAB2, kB_STATUS, kB_FIN_OFF, kB_FIN_AUX,         // batched form
   kB_QUEUE,                                                 // batched form: work-queue counters
   kG_LISTS, kG_HTAB,                                         // gather interval lists, H table
@@ -2286,15 +2286,19 @@ void rasterize(vo_context* ctx, const double* V, int64_t nv, const int32_t* F, i
   hipLaunchKernelGGL(vo::raster_bin_kernel, tgrid, dim3(256), 0, ctx->stream, dV, dF, nf, g, 1, nullptr, tcur,
                      ttris);
   check(ctx, hipGetLastError(), "raster bin launch");
-  hipLaunchKernelGGL(vo::raster_cast_kernel, dim3(unsigned(ntiles)), dim3(vo::kWave), 0, ctx->stream, dV, dF, g,
-                     toff, ttris, 0, len, nullptr, nullptr);
+  double* keep = nullptr;
+  if (ntiles <= vo::kRasterKeepTiles)
+    keep = static_cast<double*>(ws(ctx, kR_KEEP, size_t(ntiles) * vo::kRasterKeep * vo::kWave * sizeof(double)));
+  const dim3 cast_threads(vo::kWave * vo::kRasterWaves);
+  hipLaunchKernelGGL(vo::raster_cast_kernel, dim3(unsigned(ntiles)), cast_threads, 0, ctx->stream, dV, dF, g, toff, ttris,
+                     0, len, nullptr, keep, nullptr);
   check(ctx, hipGetLastError(), "raster cast launch");
   check(ctx, hipMemsetAsync(len + ncols, 0, sizeof(int64_t), ctx->stream), "memset");
   exclusive_scan(ctx, len, off, ncols + 1);
   const int64_t hits = read_word(ctx, off + ncols);
   double* dz = static_cast<double*>(ws(ctx, kR_Z, size_t(std::max<int64_t>(hits, 1)) * sizeof(double)));
-  hipLaunchKernelGGL(vo::raster_cast_kernel, dim3(unsigned(ntiles)), dim3(vo::kWave), 0, ctx->stream, dV, dF, g,
-                     toff, ttris, 1, nullptr, off, dz);
+  hipLaunchKernelGGL(vo::raster_cast_kernel, dim3(unsigned(ntiles)), cast_threads, 0, ctx->stream, dV, dF, g, toff, ttris,
+                     1, nullptr, off, keep, dz);
   check(ctx, hipGetLastError(), "raster cast launch");
   res->z.resize(size_t(hits));
   check(ctx, hipMemcpyAsync(res->off.data(), off, size_t(ncols + 1) * sizeof(int64_t), hipMemcpyDeviceToHost,
