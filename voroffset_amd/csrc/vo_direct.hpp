@@ -856,7 +856,7 @@ constexpr int direct_waves() {
 // One tile per workgroup of kSplit wavefronts.  Where only the device knows
 // how many endpoints the volume has, two launches of different splits go out
 // and the one whose range does not hold them returns at once (its 4,600 empty
-// workgroups cost 3 us at 544^2; reading the count back would cost a wait).
+// workgroups cost 4-7 us at 544^2; reading the count back would cost a wait).
 template <class T, int kList, bool kLdsTable, int kSplit>
 __global__ __launch_bounds__(kWave* kSplit, (direct_waves<kList, kSplit>())) void direct_kernel(DirectArgs<T> g) {
   __shared__ DirectSmem<T, kList> sm[kSplit];
