@@ -1,0 +1,71 @@
+"""Calls that are refused while the one-pass dilation already runs: the input
+check of a resident volume goes along with the dilation, whose kernels have to
+stay within their memory on any endpoints its offsets index."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from voroffset_amd import _native, synth
+
+from .helpers import compare_csr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = _native.Context(0)
+    yield c
+    c.close()
+
+
+def resident(off, z, prec):
+    t = torch.float32 if prec == "fp32" else torch.float64
+    d = torch.from_numpy(np.asarray(off, np.int64)).cuda(), torch.from_numpy(np.asarray(z)).to(t).cuda()
+    torch.cuda.synchronize()
+    return d
+
+
+def no_alloc(ctx, op, prec, r, nx, ny, off, z, zlo, zhi, guard=4096):
+    """The no-alloc call; returns offsets and endpoints, and looks at the words past
+    the output buffers."""
+    cap = 32 * nx * ny
+    o_off = torch.full((nx * ny + 1 + guard,), -7, dtype=torch.int64, device="cuda")
+    o_z = torch.full((cap + guard,), -7.0, dtype=z.dtype, device="cuda")
+    torch.cuda.synchronize()
+    try:
+        count, _ = ctx.morph_device_noalloc(op, prec, r, nx, ny, off.data_ptr(), z.data_ptr(), zlo, zhi, o_off.data_ptr(),
+                                            o_z.data_ptr(), cap)
+    finally:
+        torch.cuda.synchronize()
+        assert bool((o_off[nx * ny + 1:] == -7).all()) and bool((o_z[cap:] == -7.0).all())
+    return o_off[:nx * ny + 1].cpu().numpy(), o_z[:count].cpu().numpy()
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("r", [2.5, 6.5, 12.0])
+@pytest.mark.parametrize("entry", ["resident", "no_alloc"])
+def test_unsorted_columns(ctx, prec, r, entry):
+    """Many segments with their ends exchanged and in no order: 64 x 64
+    columns, four wavefronts a tile, lists of 12 in the no-alloc scratch."""
+    nx = ny = 64
+    rng = np.random.default_rng(int(10 * r))
+    k = 14
+    off = np.arange(nx * ny + 1, dtype=np.int64) * 2 * k
+    z = np.round(rng.uniform(0.0, 4000.0, 2 * k * nx * ny))
+    d_off, d_z = resident(off, z, prec)
+    with pytest.raises(_native.VoError) as e:
+        if entry == "resident":
+            ctx.morph_device("dilation", prec, r, nx, ny, d_off.data_ptr(), d_z.data_ptr(), 0.0, 4000.0)
+        else:
+            no_alloc(ctx, "dilation", prec, r, nx, ny, d_off, d_z, 0.0, 4000.0)
+    assert e.value.code == _native.ERR_ARGUMENT, str(e.value)
+    # the context, and the scratch, still work
+    vol = synth.poisson_columns(24, 20, lam=4, zmax=400, seed=3, z_margin=20)
+    d_off, d_z = resident(vol.off, vol.z, prec)
+    got = no_alloc(ctx, "dilation", prec, r, vol.nx, vol.ny, d_off, d_z, *vol.z_range())
+    seen = vol.like(vol.off, d_z.cpu().numpy().astype(np.float64))
+    bad, err = compare_csr(got[0], got[1].astype(np.float64), *oracle.morph(seen, "dilation", r))
+    assert len(bad) == 0 and err <= (1e-9 if prec == "fp64" else 1e-4)

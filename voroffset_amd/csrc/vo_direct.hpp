@@ -364,6 +364,9 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
         k += i < n && b < s ? 1 : 0;
         j += i < n && a <= e ? 1 : 0;
       }
+      // (an unsorted column's run, of a call that will be refused, may have
+      // s > e: it meets nothing, and the list stays within its room)
+      j = max(j, k);
     } else {
       // long lists: from where the last one went (runs come nearly in order)
       k = min(at, n);
@@ -374,7 +377,7 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
     }
     at = k;
     if (k == j) {
-      if (n == cap) {
+      if (n >= cap) {
         ok = 0;
         return;
       }
