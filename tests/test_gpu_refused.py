@@ -69,3 +69,21 @@ def test_unsorted_columns(ctx, prec, r, entry):
     seen = vol.like(vol.off, d_z.cpu().numpy().astype(np.float64))
     bad, err = compare_csr(got[0], got[1].astype(np.float64), *oracle.morph(seen, "dilation", r))
     assert len(bad) == 0 and err <= (1e-9 if prec == "fp64" else 1e-4)
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("r", [6.5, 12.0, 40.0])
+@pytest.mark.parametrize("side", [24, 200])
+def test_non_finite_endpoints(ctx, prec, value, r, side):
+    """Endpoints that are not numbers, among them first and last ones: waiting
+    segments without an order of their own."""
+    rng = np.random.default_rng(side)
+    k = 5
+    off = np.arange(side * side + 1, dtype=np.int64) * 2 * k
+    z = np.sort(np.round(rng.uniform(0.0, 900.0, (side * side, 2 * k)), 2), axis=1).ravel()
+    z[rng.integers(0, z.size, z.size // 7)] = value
+    d_off, d_z = resident(off, z, prec)
+    with pytest.raises(_native.VoError) as e:
+        ctx.morph_device("dilation", prec, r, side, side, d_off.data_ptr(), d_z.data_ptr(), 0.0, 900.0)
+    assert e.value.code == _native.ERR_ARGUMENT, str(e.value)

@@ -453,10 +453,13 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
       lo[t] = r < cnt2 ? float(sm.rz[first + r][0]) : NAN;
     }
     const float zmin = wave_extreme<false>(fminf(lo[0], lo[1])), zmax = wave_extreme<true>(fmaxf(lo[0], lo[1]));
-    const float scale = 33000000.f / fmaxf(zmax - zmin, 1e-20f);
+    constexpr float kKeyMax = 33000000.f;  // below 2^25
+    const float scale = kKeyMax / fmaxf(zmax - zmin, 1e-20f);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
-      key[t] = lo[t] == lo[t] ? uint32_t((lo[t] - zmin) * scale) << 7 | uint32_t(t * kWave + L) : ~0u;
+      // (every waiting segment's key holds its place, also that of a lower end
+      // that is not finite, in a call that will be refused; fmaxf drops a NaN)
+      key[t] = t * kWave + L < cnt2 ? uint32_t(fminf(fmaxf((lo[t] - zmin) * scale, 0.f), kKeyMax)) << 7 | uint32_t(t * kWave + L) : ~0u;
     sort_keys(key, cnt2 > kWave);
     for (int base = 0; base < cnt2; base += kWave) {
       const int cnt = min(cnt2 - base, kWave);
