@@ -1,6 +1,7 @@
-"""Calls that are refused while the one-pass dilation already runs: the input
-check of a resident volume goes along with the dilation, whose kernels have to
-stay within their memory on any endpoints its offsets index."""
+"""Calls that fail, and the ones after them.  The input check of a resident
+volume goes along with its one-pass dilation, whose kernels have to stay
+within their memory on any endpoints its offsets index; and a call that fails
+leaves nothing behind that a later one takes for its own."""
 
 import numpy as np
 import pytest
@@ -87,3 +88,32 @@ def test_non_finite_endpoints(ctx, prec, value, r, side):
     with pytest.raises(_native.VoError) as e:
         ctx.morph_device("dilation", prec, r, side, side, d_off.data_ptr(), d_z.data_ptr(), 0.0, 900.0)
     assert e.value.code == _native.ERR_ARGUMENT, str(e.value)
+
+
+@pytest.mark.parametrize("form", ["one pass", "two sweeps"])
+def test_growth_table_after_a_failure(monkeypatch, form):
+    """A call fails (injected) where its larger radius has the context give
+    the growth table's memory back for more; the earlier radius follows."""
+    monkeypatch.setenv("VO_INJECT_HIP_ERROR", "hipFree")
+    if form == "two sweeps":
+        monkeypatch.setenv("VO_PASS1", "zsweep")
+    c = _native.Context(0)
+    monkeypatch.undo()
+    nx, ny = 3, 2  # (few enough endpoints that no other buffer grows)
+    off, z = [0, 2, 2, 2, 2, 2, 2], np.array([10.0, 20.0])
+    d_off, d_z = resident(off, z, "fp64")
+
+    def dilated(r):
+        out, count, _ = c.morph_device("dilation", "fp64", r, nx, ny, d_off.data_ptr(), d_z.data_ptr(), 0.0, 100.0)
+        return _native.to_host(out.z, np.float64, count).reshape(-1, 2)
+
+    try:
+        want = [[10.0 - h, 20.0 + h] for y in range(ny) for x in range(nx) for h in [np.sqrt(4.5 * 4.5 - x * x - y * y)]]
+        assert np.array_equal(dilated(4.5), want)
+        for _ in range(3):
+            with pytest.raises(_native.VoError) as e:
+                dilated(30.5)
+            assert e.value.code == _native.ERR_DEVICE and "injected" in str(e.value)
+            assert np.array_equal(dilated(4.5), want)
+    finally:
+        c.close()

@@ -225,14 +225,12 @@ struct vo_context {
   int num_cus = 0;                // compute units of the device
   std::map<std::pair<const void*, size_t>, int> resident;  // workgroups per CU, by kernel and dynamic LDS
   int last_fallback_tiles = 0;
-  // the radius whose gather table the H-table slot holds, and where (a call
+  // the radius whose gather table the H-table slot holds (-1: none; a call
   // with the same radius skips the upload)
   double htab_R = -1;
-  const void* htab_at = nullptr;
   // the same for the one-pass form's table and block order
   double dtab_R = -1;
   int dtab_axis = 0;
-  const void* dtab_at = nullptr;
   int dtab_norder = 0;
   bool two_pass = false;  // VO_PASS1=zsweep, vo_pass1, vo_autotune: keep to the two sweeps
   int direct_cap = 24;    // intervals per list of the one-pass form (grows on overflow)
@@ -332,11 +330,15 @@ void* ws(vo_context* ctx, int slot, size_t bytes) {
   Buffer& b = ctx->buf[slot];
   if (bytes == 0) bytes = 16;
   if (b.bytes < bytes) {
+    // what a slot held goes with it, whatever of this call fails from here on
+    if (slot == kD_TAB) ctx->dtab_R = -1;
+    if (slot == kG_HTAB) ctx->htab_R = -1;
     if (b.ptr) {
       check(ctx, hipStreamSynchronize(ctx->stream), "sync");  // the old buffer may still be in use
-      check(ctx, hipFree(b.ptr), "hipFree");
+      void* old = b.ptr;
+      b = Buffer();
+      check(ctx, hipFree(old), "hipFree");
     }
-    b.ptr = nullptr;
     const size_t want = bytes + bytes / 4;
     if (hipMalloc(&b.ptr, want) != hipSuccess) {
       b.ptr = nullptr;
@@ -418,21 +420,20 @@ void append_htab(double R, std::vector<double>& out) {
 // values alive until the upload has run (the caller synchronises before it
 // goes out of scope).  Returns the device base.
 // A table already in place for the same single radius (the slot is written
-// by nothing else and is reallocated only to grow, that is for another
-// radius) is not uploaded again; the no-alloc scratch is shared by other
+// by nothing else, and ws() forgets the table where it moves the slot) is not
+// uploaded again; the no-alloc scratch is shared by other
 // calls, so there the table is always uploaded.
 const double* upload_htab(vo_context* ctx, int slot, const std::vector<double>& radii, std::vector<double>& host) {
   host.clear();
   for (double R : radii) append_htab(R, host);
   double* d = static_cast<double*>(ws(ctx, slot, host.size() * sizeof(double)));
-  const bool cached = !ctx->arena.on && radii.size() == 1 && radii[0] == ctx->htab_R && d == ctx->htab_at;
+  const bool cached = !ctx->arena.on && radii.size() == 1 && radii[0] == ctx->htab_R;
   if (!cached) {
     ctx->htab_R = -1;  // (until the upload is in the stream)
     check(ctx, hipMemcpyAsync(d, host.data(), host.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream),
           "upload H table");
     if (!ctx->arena.on && radii.size() == 1) {
       ctx->htab_R = radii[0];
-      ctx->htab_at = d;
     }
   }
   return d;
@@ -657,10 +658,12 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   const int sparse_split = in.count >= 0 || ctx->arena.on ? split : direct_split(ntiles, 0, sparse, rint);
   const int W = vo::direct_htab_width(rint);
   DirectTable tab;  // outlives its upload (a synchronisation follows)
-  const bool cached = !ctx->arena.on && ctx->dtab_R == R && ctx->dtab_axis == int(along_x) && ctx->dtab_at;
+  // (ws() forgets the table with its slot, which moves only to grow: never for
+  // the radius it holds)
+  const bool cached = !ctx->arena.on && ctx->dtab_R == R && ctx->dtab_axis == int(along_x);
   if (!cached) tab = direct_table(R, along_x);
   const size_t hbytes = size_t(W) * W * sizeof(double);
-  int norder = cached ? ctx->dtab_norder : int(tab.order.size());
+  const int norder = cached ? ctx->dtab_norder : int(tab.order.size());
   const size_t tbytes = hbytes + size_t(norder) * sizeof(int2);
   auto list_bytes = [&](int64_t tiles, int c) {
     const int sparse_lds = direct_list(rint, sparse_split);
@@ -707,8 +710,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   }
   hipLaunchKernelGGL(vo::reset_words_kernel, dim3(1), dim3(1), 0, ctx->stream, status, tiles, o_len + ncols, chk_word);
   check(ctx, hipGetLastError(), "reset words");
-  if (!cached || dtab != ctx->dtab_at) {
-    if (cached) tab = direct_table(R, along_x);
+  if (!cached) {
     ctx->dtab_R = -1;  // (until the upload is in the stream)
     check(ctx, hipMemcpyAsync(dtab, tab.h.data(), hbytes, hipMemcpyHostToDevice, ctx->stream), "upload H table");
     check(ctx, hipMemcpyAsync(dtab + hbytes, tab.order.data(), tab.order.size() * sizeof(int2), hipMemcpyHostToDevice,
@@ -717,7 +719,6 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
     if (!ctx->arena.on) {
       ctx->dtab_R = R;
       ctx->dtab_axis = int(along_x);
-      ctx->dtab_at = dtab;
       ctx->dtab_norder = norder;
     }
   }
@@ -2136,6 +2137,15 @@ void autotune(vo_context* ctx, const vo_volume* sample, int n, const double* rad
   }
 }
 
+// A call that failed leaves no input check behind, and what it was writing on
+// the device is not relied on.
+void forget_after_failure(vo_context* ctx) {
+  ctx->check_input = false;
+  ctx->fused.word = nullptr;
+  ctx->chain_dirty = true;
+  ctx->htab_R = ctx->dtab_R = -1;
+}
+
 int guarded(vo_context* ctx, const std::function<void()>& body) {
   if (!ctx) return VO_ERR_ARGUMENT;
   // a call's input check never outlives it
@@ -2149,14 +2159,10 @@ int guarded(vo_context* ctx, const std::function<void()>& body) {
     ctx->fused.word = nullptr;
     return VO_OK;
   } catch (const Failure& f) {
-    ctx->check_input = false;
-    ctx->fused.word = nullptr;
-    ctx->chain_dirty = true;
+    forget_after_failure(ctx);
     return f.code;
   } catch (const std::exception& e) {
-    ctx->check_input = false;
-    ctx->fused.word = nullptr;
-    ctx->chain_dirty = true;
+    forget_after_failure(ctx);
     ctx->error = e.what();
     return VO_ERR_ARGUMENT;
   }
