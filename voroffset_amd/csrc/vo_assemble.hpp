@@ -137,8 +137,15 @@ __device__ void assemble(int64_t n, int64_t* off, int64_t cap, const AssembleSta
     }
   }
   // the last workgroup to come here leaves everything zero: nobody looks at
-  // the sums any more
-  if (threadIdx.x == 0) s_block = atomicAdd(&st.ticket[1], 1u);
+  // the sums any more, and none is still on its way: the wavefront that
+  // published this workgroup's waits for the store's completion (an agent-scope
+  // store completes where every XCD sees it) before it counts itself done.
+  // Without the wait the two words are not ordered, and a late sum would stay
+  // for the next launch to take for its own.
+  if (threadIdx.x == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    s_block = atomicAdd(&st.ticket[1], 1u);
+  }
   __syncthreads();
   if (s_block == gridDim.x - 1) {
     for (unsigned i = threadIdx.x; i < gridDim.x; i += kAssembleThreads) st.sum[i] = 0;
