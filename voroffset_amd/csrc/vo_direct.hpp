@@ -14,6 +14,7 @@
 // bit.
 #pragma once
 
+#include <cfloat>
 #include <type_traits>
 
 #include "vo_sweeps.hpp"
@@ -209,14 +210,16 @@ __device__ __forceinline__ float wave_extreme(float v) {
   step(std::integral_constant<int, 0x143>{});
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), kWave - 1));
 }
-// a double as a float at or above / at or below it
+// A double as a float at or above / at or below it.  Past the largest float
+// that is the largest one on the side towards zero and infinity on the other;
+// the last term is what floats too small to have a rounding step are off by.
 __device__ __forceinline__ float float_up(double v) {
-  const float f = float(v);
-  return f + fabsf(f) * 2.4e-7f;
+  const float f = fmaxf(float(v), -FLT_MAX);
+  return f + fmaf(fabsf(f), 2.4e-7f, 1e-37f);
 }
 __device__ __forceinline__ float float_down(double v) {
-  const float f = float(v);
-  return f - fabsf(f) * 2.4e-7f;
+  const float f = fminf(float(v), FLT_MAX);
+  return f - fmaf(fabsf(f), 2.4e-7f, 1e-37f);
 }
 // The smaller / larger of this lane's value and the one of lane L ^ D, in
 // registers (no LDS round trip).
