@@ -1,0 +1,101 @@
+"""Which form a dilation takes depends on the radius, the tiles and the
+endpoints per column: on both sides of each line of the rule the default
+context gives what the two sweeps give (VO_PASS1=zsweep), bit for bit, for
+volumes whose size the host knows and for those it has to ask the device."""
+
+import numpy as np
+import pytest
+import torch
+
+from voroffset_amd import _native
+from voroffset_amd.volume import CompressedVolume
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def contexts():
+    one = _native.Context(0)
+    with pytest.MonkeyPatch.context() as m:
+        m.setenv("VO_PASS1", "zsweep")
+        two = _native.Context(0)
+    yield one, two
+    one.close()
+    two.close()
+
+
+def volume(nx, ny, segments, seed, zext=400.0, margin=12.0):
+    """About `segments` segments a column, some columns empty, some touching or of no length."""
+    rng = np.random.default_rng(seed)
+    k = rng.poisson(segments, nx * ny)
+    off = np.zeros(nx * ny + 1, np.int64)
+    np.cumsum(2 * k, out=off[1:])
+    col = np.repeat(np.arange(nx * ny), 2 * k)
+    z = rng.integers(0, int(16 * zext), col.size)
+    z = z[np.lexsort((z, col))] / 16.0
+    return CompressedVolume(nx, ny, off, z, origin=(0.0, 0.0, -margin), extent=(float(nx), float(ny), zext + 2 * margin),
+                            spacing=1.0, padding=0)
+
+
+def same(contexts, vol, op, prec, r):
+    zlo, zhi = vol.z_range()
+    res = [c.morph_host(op, prec, r, vol.nx, vol.ny, vol.off, vol.z, zlo, zhi)[:2] for c in contexts]
+    assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
+    # the same on the device, relative to the shift that host volumes travel with
+    shift = _native.storage_shift(zlo, zhi) if prec == "fp32" else 0.0
+    t = torch.float32 if prec == "fp32" else torch.float64
+    off, z = torch.from_numpy(vol.off).cuda(), torch.from_numpy(vol.z - shift).to(t).cuda()
+    z = z if z.numel() else torch.zeros(1, dtype=t, device="cuda")
+    torch.cuda.synchronize()
+    out, count, _ = contexts[0].morph_device(op, prec, r, vol.nx, vol.ny, off.data_ptr(), z.data_ptr(), zlo - shift,
+                                             zhi - shift)
+    assert np.array_equal(_native.to_host(out.offsets, np.int64, out.nx * out.ny + 1), res[0][0])
+    got = _native.to_host(out.z, np.float32 if prec == "fp32" else np.float64, count)
+    assert np.array_equal(got.astype(np.float64) + shift, res[0][1])
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("nx,ny", [(3, 5), (9, 2), (32, 32), (33, 32), (256, 128), (257, 128)])
+@pytest.mark.parametrize("segments", [1, 4, 10, 24, 45])
+@pytest.mark.parametrize("r", [0.5, 1.9, 2.5, 3.0, 4.5, 5.9, 6.0])
+def test_lines_of_the_rule(contexts, prec, nx, ny, segments, r):
+    if nx * ny * segments > 800_000:
+        pytest.skip("kept small")
+    same(contexts, volume(nx, ny, segments, nx + segments), "dilation", prec, r)
+
+
+@pytest.mark.parametrize("nx,ny", [(384, 256), (385, 256), (768, 256), (769, 256), (1024, 384), (1025, 384)])
+@pytest.mark.parametrize("segments", [0.4, 1.5, 2.5])
+@pytest.mark.parametrize("op,r", [("dilation", 2.0), ("dilation", 3.5), ("dilation", 4.0), ("dilation", 5.0),
+                                  ("dilation", 15.9), ("dilation", 16.0), ("closing", 4.0), ("closing", 5.5)])
+def test_shared_tiles(contexts, nx, ny, segments, op, r):
+    same(contexts, volume(nx, ny, segments, int(r) + nx, zext=250.0), op, "fp32", r)
+
+
+@pytest.mark.parametrize("op", ["erosion", "closing", "opening"])
+@pytest.mark.parametrize("segments", [3, 14, 20])
+@pytest.mark.parametrize("r", [0.7, 1.5, 2.2, 4.0])
+def test_complements(contexts, op, segments, r):
+    same(contexts, volume(61, 47, segments, segments), op, "fp32", r)
+
+
+def test_taken_after_the_sweeps_refuse(contexts):
+    """A volume the rule gives to the sweeps, with one column of more segments
+    than their windows take: the one-pass form does it."""
+    nx, ny, n = 90, 60, 70000
+    vol = volume(nx, ny, 4, 1)
+    cols = [vol.z[a:b] for a, b in zip(vol.off[:-1], vol.off[1:])]
+    at = 30 * nx + 40
+    cols[at] = np.arange(2 * n) * 0.5
+    vol = CompressedVolume.from_columns(nx, ny, [c.tolist() for c in cols], origin=(0.0, 0.0, -10.0),
+                                        extent=(float(nx), float(ny), n + 20.0))
+    zlo, zhi = vol.z_range()
+    args = ("dilation", "fp64", 2.5, nx, ny, vol.off, vol.z, zlo, zhi)
+    with pytest.raises(_native.VoError) as e:
+        contexts[1].morph_host(*args)
+    assert e.value.code == _native.ERR_CAPACITY
+    for _ in range(2):
+        off, z, _ = contexts[0].morph_host(*args)
+        h = np.sqrt(2.5 * 2.5 - 1.0)
+        assert z[off[at + 1]] == min(0.0, z[off[at + 1]]) and z[off[at]] <= -2.5
+        assert z[off[at + 1] + 1] == n - 0.5 + h and z[off[at] + 1] == n - 0.5 + 2.5

@@ -59,32 +59,84 @@ struct Tuning {
   int events[kTuneBuckets] = {768, 768, 768, 768, 768};
   int ocap[kTuneBuckets] = {24, 16, 16, 16, 16};
 };
-// pass-1 z-sweep form: LDS events per z-slab (denser windows take more slabs)
-// and histogram bins; small enough for ~5 waves per SIMD
-// One-pass form: few tiles leave most of the card idle, each a long serial
-// chain: up to 512 of them four wavefronts share a tile (86 x 88 solids at
-// R = 6.4: 400 -> 191 us, 212 x 118 closing at R = 27: 466 -> 171, 64 x 48 at
-// R = 4: 255 -> 228; above, the wavefronts' weaker covers cost more than they
-// give: 216 x 310 at R = 2, 1053 tiles, 340 -> 513).
-// Where the volume holds few segments per column (the host knows, or the
-// kernels look: see direct_kernel) there is little cover to lose, and at radii
-// below 16 two wavefronts a tile shorten the tail of up to 6144 tiles: 544^2
-// tubes at R = 10 687 -> 623 us, 336^2 tubes closed at R = 3 291 -> 214 in the last
-// dilation, 512^2 solids at R = 4 295 -> 280.  Denser columns lose (1531 x 219 at
-// R = 7.3, 5 endpoints a column, 234 -> 316; 839 x 339 at R = 4.8, 6.4 of them,
-// 360 -> 503), and so do large radii (1097 x 310 solids at R = 35 698 -> 758).  A
-// complement's columns have two endpoints more, and what the dilation before
-// it parted: four more are allowed (the last dilation of 544^2 tubes closed
-// at R = 5 910 -> 720; the other side is an erosion of 1531 x 219 short random
-// segments, 78 -> 131).
-constexpr int kDirectSplitTiles = 512, kDirectSplitSparseTiles = 6144;
-constexpr int64_t kDirectSparse = 4;  // endpoints per column
-constexpr int kDirectSparseR = 16;
-constexpr int64_t direct_sparse(int64_t ncols, bool outer) { return (kDirectSparse + 4 * outer) * ncols; }
-inline int direct_split(int64_t ntiles, int64_t endpoints, int64_t sparse, int rint) {
-  if (ntiles <= kDirectSplitTiles) return 4;
-  return ntiles <= kDirectSplitSparseTiles && rint < kDirectSparseR && endpoints >= 0 && endpoints <= sparse ? 2 : 1;
+// --- the form a dilation takes -----------------------------------------------
+// By the radius, the tiles (n, of 8 x 8 columns) and the endpoints a column (e).
+// Figures are whole calls in us, or ratios to the two sweeps, on random
+// segments in HBM unless they say otherwise.
+//
+// The one-pass form is the faster one at radii from 6 on wherever it was
+// measured (256^2, R = 8: e = 12 267 -> 123, e = 120 2835 -> 714).  Below, a lane's own
+// columns come in before anything covers them, and the length its list goes
+// through decides:
+//   R < 1: a column is alone.  e = 6-12 1.07-1.3, e = 40-120 0.63-0.75.
+//   R < 2: 5 or 9 columns meet, few fuse.  e up to 40 0.6-1.2, e = 80 1.2-2.4, e = 140
+//     and more 2-3.9; at 25 tiles e = 4 1.0, e = 6 1.1, e = 14 1.5.
+//   R < sqrt(5), 13 columns: up to 1536 tiles e = 14 1.0-1.1, e = 28 1.35-1.5, e = 300
+//     1.7-2.3; above them 0.65-1.25.  At 36 tiles e = 12 1.15-1.25.
+//   R < 3: 0.56-1.07 above 48 tiles, but 1.65 on 64^2 of 60 equal layers; up to
+//     48 tiles e = 18-40 1.1-2.
+//   R < 4: 0.62-1.05 above 16 tiles, up to those e = 28-40 1.1-2.
+//   R < 5: e = 24 0.85-1.03 up to 1024 tiles and 1.17-1.19 above, e = 40 1.0-1.3 and
+//     1.5, e = 120 1.5-2.3; up to 16 tiles e = 18-40 0.9-2.
+//   R < 6: e = 40 0.7-0.95 up to 1024 tiles and 0.9-1.2 above, e = 200 1.7-2.9.
+// Grids so thin that most of a tile is outside waste it where the work is
+// little (100000 x 2, e = 12, R = 2: 302 -> 458; R = 16: 339 -> 202).  Columns that a
+// ring complement ends in have long segments outside (erosion of 256^2, e = 14,
+// R = 2: 390 -> 325; e = 82 2866 -> 3259).
+constexpr int kSharedTiles = 512, kPairedMidTiles = 3072, kPairedSparseTiles = 6144;
+constexpr int64_t kSparse = 4;  // endpoints per column
+struct Load {                   // what the rules look at
+  int64_t ncols, ntiles, endpoints;  // (endpoints -1: not known)
+  bool outer;                        // columns end in the segments of a ring complement
+  bool wide;                         // FP64 endpoints
+  bool above(double e) const { return double(endpoints) > e * double(ncols); }
+  Load of(int64_t e) const { return Load{ncols, ntiles, e, outer, wide}; }
+  int64_t sparse() const { return (kSparse + (outer ? 4 : 0)) * ncols; }
+};
+inline bool prefers_sweeps(const Load& v, double R) {
+  // (a few columns are launches and waits; those of more than 400 the sweeps refuse, after a look at all of them)
+  if (v.ncols <= 16 || v.above(400)) return false;
+  const int64_t n = v.ntiles;
+  if (R < 1) return !v.outer && v.above(kSparse) && !v.above(16);
+  if (v.outer && R < 3) return v.above(64);
+  if (R < 3 && v.ncols < n * (vo::kWave / 2)) return v.above(kSparse);
+  if (R < 2) return v.above(n <= 36 ? 5 : 64);
+  if (R * R < 5) return v.above(n <= 36 ? 8 : (n <= 1536 ? 16 : 160));
+  if (R < 3) return n <= kSharedTiles && v.above(n <= 48 ? 16 : 100);
+  if (R < 4) return n <= 16 && v.above(24);
+  if (R < 5) return v.above(n > 16 && n <= 1024 ? 32 : 16);
+  if (R < 6) return v.above(n <= 1024 ? 64 : 40);
+  return false;
 }
+// Wavefronts that share a tile.  Few tiles leave most of the card idle, each a
+// long serial chain: up to 512 four of them do (86 x 88 solids at R = 6.4: 400
+// -> 191, 212 x 118 closing at R = 27: 466 -> 171), below R = 4 only sparse ones (139 x
+// 121 solids eroded at R = 2.4: 238, with two 282), else two: lists are long and want
+// the whole cover (64^2, e = 12, R = 3: 0.82, 0.76 and 0.92 times the sweeps for one,
+// two and four); those of dense columns are not shared (64^2, e = 80: R = 2 1.3, 3.1 and 3.2; R = 1.5 1.2, 2.3 and
+// 1.9).  Up to as many tiles as are resident together two share one (kernel,
+// 270^2, e = 4: R = 2 180 -> 144, R = 4 191 -> 132, R = 8 123 -> 87; 256^2 at R = 20 0.77-0.98 of
+// one, but R = 100 1.07 and R = 200 1.15; 360^2, 2025
+// tiles, 1.1-1.2; FP64, of which fewer are resident: 280^2, 1225 tiles, R = 2.5 1.2-1.4).
+// Above, the wavefronts' weaker covers cost more than they give (kernel, 512^2,
+// e = 2: 1.4-1.6 times), except on the tails that filigree and solids have: for
+// columns of few endpoints (a ring complement has two more, and what the
+// dilation before it parted: four are allowed) and radii from 3 to 16, two up to 6144 tiles
+// (kernel, tubes, R = 4 / 8: 400^2 266 -> 163, 418 -> 256; 512^2 306 -> 282, 526 -> 465; closed
+// at R = 5 892 -> 776).  Past 3072 tiles that gain begins at R = 5, at R = 4 for the
+// sparsest (kernel: 512^2 solids closed at R = 4 456 -> 525, tubes as above), before
+// them at R = 3 (300^2 tubes 180 -> 153; closed at R = 1 149 -> 166).
+inline int direct_split(const Load& v, double R) {
+  const int64_t n = v.ntiles;
+  const bool dense = v.endpoints > v.sparse();
+  if (R < 4 && v.above(R < 1 ? 16 : (R < 2 ? 48 : (R < 3 ? 20 : 100)))) return 1;
+  if (n <= kSharedTiles) return R < 4 && dense ? 2 : 4;
+  if (n <= (v.wide ? 1024 : 1536)) return R < 64 && (R >= 6 || !v.above(48)) ? 2 : 1;
+  if (R < 3 || R >= 16 || n > kPairedSparseTiles || dense) return 1;
+  return n <= kPairedMidTiles || R >= 5 || (R >= 4 && !v.outer && !v.above(1.5)) ? 2 : 1;
+}
+// Whether the host has to know the endpoints (for the form, and small radii's splits).
+inline bool rules_count(double R) { return R < 6; }
 // Entries of a lane's interval list kept in LDS: the long list where columns
 // keep several intervals (small radii) or LDS does not decide how many waves
 // fit (split tiles), the short one elsewhere.
@@ -92,6 +144,8 @@ constexpr int kDirectListLong = 8, kDirectListShort = 3, kDirectSmallR = 3;
 inline int direct_list(int rint, int split) {
   return split > 1 || rint <= kDirectSmallR ? kDirectListLong : kDirectListShort;
 }
+// pass-1 z-sweep form: LDS events per z-slab (denser windows take more slabs)
+// and histogram bins; small enough for ~5 waves per SIMD
 constexpr int kZECap = 768, kZNB = 512, kZWMax = 64 + 2 * 128, kZWMax8 = 64 + 2 * 256;
 
 template <class T>
@@ -158,7 +212,7 @@ struct DevVol {
   int nx = 0, ny = 0;
   const int64_t* off = nullptr;
   const void* z = nullptr;
-  int64_t count = 0;     // endpoints (-1: not known on the host)
+  int64_t count = -1;    // endpoints (-1: not known on the host)
   bool outer = false;    // columns end in two endpoints that a ring complement added
   bool pending = false;  // the count is in host_words[4] after the next synchronisation
 };
@@ -233,6 +287,7 @@ struct vo_context {
   int dtab_axis = 0;
   int dtab_norder = 0;
   bool two_pass = false;  // VO_PASS1=zsweep, vo_pass1, vo_autotune: keep to the two sweeps
+  bool asked_sweeps = false;  // what the last device-held volume whose size was asked for took
   int direct_cap = 24;    // intervals per list of the one-pass form (grows on overflow)
   bool chain_dirty = false;  // a call failed: the chained scan's words may not be zero
   int64_t spec_out = 0;  // endpoints the next dilation's output is first sized for
@@ -386,6 +441,33 @@ int64_t read_word(vo_context* ctx, const int64_t* dptr) {
         "copy word");
   sync(ctx);
   return ctx->host_words[0];
+}
+
+// The endpoints of a volume that only the device knows: reset_words_kernel
+// writes them to host_words[7] (the other words have writers of their own),
+// asked for before its launch, awaited when the kernels that do not depend on
+// them are in the stream too.
+constexpr int64_t kCountPending = -1;
+int64_t* ask_count(vo_context* ctx) {
+  __atomic_store_n(ctx->host_words + 7, kCountPending, __ATOMIC_RELEASE);
+  return ctx->host_words + 7;
+}
+int64_t await_count(vo_context* ctx) {
+  int64_t n = kCountPending;
+  for (unsigned spins = 1; (n = __atomic_load_n(ctx->host_words + 7, __ATOMIC_ACQUIRE)) == kCountPending; ++spins) {
+    if (spins % 65536 != 0) continue;
+    // an error, or a stream that ran dry, ends the wait
+    const hipError_t e = hipStreamQuery(ctx->stream);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    check(ctx, e, "await count");
+    n = __atomic_load_n(ctx->host_words + 7, __ATOMIC_ACQUIRE);
+    if (n == kCountPending) fail(ctx, VO_ERR_DEVICE, "await count: the stream ended without it");
+    break;
+  }
+  return n;
 }
 
 std::string status_text(int s) {
@@ -636,26 +718,32 @@ void launch_direct_batch(vo_context* ctx, int c, int max_rint, const vo::DirectA
 }
 
 // One dilation in one pass (vo_direct.hpp): returns false, with nothing done,
-// where the two sweeps have to take it (no room in the no-alloc scratch, or
-// lists past
-// kDirectMaxList or kGatherRoomBytes).  `chk` is a pending input check (word null:
-// none), done by the summary kernel.
+// where the two sweeps have to take it or are the faster form (prefers_sweeps;
+// no room in the no-alloc scratch; lists past kDirectMaxList or
+// kGatherRoomBytes).  `chk` is a pending input check (word null: none), done
+// by the summary kernel.
 template <class T>
 bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, const vo::InputCheck<T>& chk, int* chk_word,
-                   int64_t* out_off, int out_z_slot, DevVol& out, double* t1, double* t2) {
+                   int64_t* out_off, int out_z_slot, DevVol& out, double* t1, double* t2, bool* by_rule) {
   const int rint = int(std::floor(R));
   const int nbx = (in.nx + vo::kSide - 1) / vo::kSide, nby = (in.ny + vo::kSide - 1) / vo::kSide;
   const int64_t ncols = int64_t(in.nx) * in.ny, ntiles = int64_t(nbx) * nby;
   if (ntiles * vo::kWave > INT32_MAX) return false;
+  Load load{ncols, ntiles, in.count, in.outer, sizeof(T) == 8};
+  const bool ask = in.count < 0 && rules_count(R);
+  auto sweeps = [&] {  // chosen for their speed
+    const bool s = by_rule && load.endpoints >= 0 && prefers_sweeps(load, R);
+    if (s) *by_rule = true;
+    return s;
+  };
+  if (sweeps()) return false;
+  // the answer to `ask` is awaited with the summary in the stream, which takes
+  // longer than it; if the last one was the sweeps, before the summary
+  const bool early = ask && ctx->asked_sweeps;
   const bool along_x = ax.sy == 1;
   int* status = static_cast<int*>(slot_ptr(ctx, kSTATUS));
   int64_t* o_start = static_cast<int64_t*>(slot_ptr(ctx, kO_START));
   int64_t* o_len = static_cast<int64_t*>(slot_ptr(ctx, kO_LEN));
-  int cap = ctx->direct_cap;
-  const int64_t sparse = direct_sparse(ncols, in.outer);
-  const int split = direct_split(ntiles, in.count, sparse, rint), in_lds = direct_list(rint, split);
-  // (the split a sparse volume would take, where only the device knows)
-  const int sparse_split = in.count >= 0 || ctx->arena.on ? split : direct_split(ntiles, 0, sparse, rint);
   const int W = vo::direct_htab_width(rint);
   DirectTable tab;  // outlives its upload (a synchronisation follows)
   // (ws() forgets the table with its slot, which moves only to grow: never for
@@ -665,17 +753,10 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   const size_t hbytes = size_t(W) * W * sizeof(double);
   const int norder = cached ? ctx->dtab_norder : int(tab.order.size());
   const size_t tbytes = hbytes + size_t(norder) * sizeof(int2);
-  auto list_bytes = [&](int64_t tiles, int c) {
-    const int sparse_lds = direct_list(rint, sparse_split);
-    return size_t(tiles) * std::max(split * (c - in_lds), sparse_split * (c - sparse_lds)) * 2 * vo::kWave * sizeof(double);
-  };
-  auto out_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * 2 * c * vo::kWave * sizeof(T); };
   vo::Ends<T>*col, *blk;
   uint64_t* at;
   int *bcnt, *tiles;
   char* dtab;
-  T* o_z;
-  double* spill;
   if (ctx->arena.on) {
     // the sweeps' buffers are reserved already; this form's go inside them
     size_t used = 0;
@@ -693,11 +774,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
     bcnt = reinterpret_cast<int*>(take(size_t(ntiles) * sizeof(int)));
     tiles = reinterpret_cast<int*>(take(size_t(ntiles + 1) * sizeof(int)));
     dtab = take(tbytes);
-    const Buffer &lists = ctx->arena.slot[kG_LISTS], &oz = ctx->arena.slot[kO_Z];
-    cap = int(std::min(std::min(size_t(cap), oz.bytes / out_bytes(ntiles, 1)), in_lds + lists.bytes / list_bytes(ntiles, in_lds + 1)));
-    if (!fits || cap < 12) return false;
-    spill = static_cast<double*>(lists.ptr);
-    o_z = static_cast<T*>(oz.ptr);
+    if (!fits) return false;
   } else {
     col = static_cast<vo::Ends<T>*>(ws(ctx, kD_COL, size_t(ntiles) * vo::kWave * sizeof(vo::Ends<T>)));
     at = static_cast<uint64_t*>(ws(ctx, kD_AT, size_t(ntiles) * vo::kWave * sizeof(uint64_t)));
@@ -705,11 +782,15 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
     bcnt = static_cast<int*>(ws(ctx, kD_BCNT, size_t(ntiles) * sizeof(int)));
     tiles = static_cast<int*>(ws(ctx, kTILES, size_t(2 * ntiles + 2) * sizeof(int)));
     dtab = static_cast<char*>(ws(ctx, kD_TAB, tbytes));
-    spill = static_cast<double*>(ws(ctx, kG_LISTS, list_bytes(ntiles, cap)));
-    o_z = static_cast<T*>(ws(ctx, kO_Z, out_bytes(ntiles, cap)));
   }
-  hipLaunchKernelGGL(vo::reset_words_kernel, dim3(1), dim3(1), 0, ctx->stream, status, tiles, o_len + ncols, chk_word);
+  hipLaunchKernelGGL(vo::reset_words_kernel, dim3(1), dim3(1), 0, ctx->stream, status, tiles, o_len + ncols, chk_word, in.off,
+                     ncols, ask ? ask_count(ctx) : nullptr);
   check(ctx, hipGetLastError(), "reset words");
+  auto answer = [&] {
+    load.endpoints = await_count(ctx);
+    return ctx->asked_sweeps = sweeps();
+  };
+  if (early && answer()) return false;
   if (!cached) {
     ctx->dtab_R = -1;  // (until the upload is in the stream)
     check(ctx, hipMemcpyAsync(dtab, tab.h.data(), hbytes, hipMemcpyHostToDevice, ctx->stream), "upload H table");
@@ -731,6 +812,42 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
     check(ctx, hipGetLastError(), "pass1 launch");
   }
   check(ctx, hipEventRecord(ctx->ev[1], ctx->stream), "event");
+  auto give_up = [&] {
+    if (!cached) check(ctx, hipStreamSynchronize(ctx->stream), "sync");  // the table's upload
+    return false;
+  };
+  if (ask && !early && answer()) return give_up();
+  // (where only the device knows the endpoints, the splits of a volume above and up to the line)
+  const bool known = load.endpoints >= 0 || ctx->arena.on;
+  int split = direct_split(known ? load : load.of(load.sparse() + 1), R), in_lds = direct_list(rint, split);
+  int sparse_split = known ? split : direct_split(load.of(load.sparse()), R);
+  int cap = ctx->direct_cap;
+  auto list_bytes = [&](int64_t tiles, int c) {
+    const int sparse_lds = direct_list(rint, sparse_split);
+    return size_t(tiles) * std::max(split * (c - in_lds), sparse_split * (c - sparse_lds)) * 2 * vo::kWave * sizeof(double);
+  };
+  auto out_bytes = [&](int64_t tiles, int c) { return size_t(tiles) * 2 * c * vo::kWave * sizeof(T); };
+  T* o_z;
+  double* spill;
+  if (ctx->arena.on) {
+    const Buffer &lists = ctx->arena.slot[kG_LISTS], &oz = ctx->arena.slot[kO_Z];
+    auto room = [&] {
+      return int(std::min(std::min(size_t(cap), oz.bytes / out_bytes(ntiles, 1)), in_lds + lists.bytes / list_bytes(ntiles, in_lds + 1)));
+    };
+    // (wavefronts that share a tile share its room too: lists of 12 to 14 instead
+    // of 20 sent 128^2, e = 20, at R = 4 on to the sweeps, 313 -> 675 us)
+    while (R < 6 && split > 1 && room() < 16) {
+      sparse_split = split /= 2;
+      in_lds = direct_list(rint, split);
+    }
+    cap = room();
+    if (cap < 12) return give_up();
+    spill = static_cast<double*>(lists.ptr);
+    o_z = static_cast<T*>(oz.ptr);
+  } else {
+    spill = static_cast<double*>(ws(ctx, kG_LISTS, list_bytes(ntiles, cap)));
+    o_z = static_cast<T*>(ws(ctx, kO_Z, out_bytes(ntiles, cap)));
+  }
   vo::DirectArgs<T> a{in.nx, in.ny, nbx, nby, rint, in.off, z, col, at, blk, bcnt,
                       reinterpret_cast<const double*>(dtab), reinterpret_cast<const int2*>(dtab + hbytes), norder,
                       o_z, int64_t(2) * cap * vo::kWave, 0, o_start, o_len, cap, spill, tiles, status, nullptr};
@@ -740,7 +857,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   for (;;) {
     if (sparse_split != split) {
       a.least = INT64_MIN;
-      a.most = sparse;
+      a.most = load.sparse();
       launch_direct<T>(ctx, rint, sparse_split, a, int(todo));
       check(ctx, hipGetLastError(), "pass2 gather launch");
       a.least = a.most + 1;
@@ -836,10 +953,11 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   return true;
 }
 
-// One dilation: `in` -> CSR in (out_off_slot, out_z_slot).
+// One dilation: `in` -> CSR in (out_off_slot, out_z_slot).  Where the sweeps are
+// free to be chosen (`by_rule`), it says so if they were.
 template <class T>
-DevVol dilate(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int out_z_slot, double* t1,
-              double* t2) {
+DevVol dilate_as(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int out_z_slot, double* t1, double* t2,
+                 bool* by_rule) {
   // the passes work on a logical grid of nx lines of ny positions: pass 1
   // sweeps along the positions of each line, pass 2 across the lines
   const Axis ax = axis_for(ctx, in.nx, in.ny);
@@ -868,6 +986,7 @@ DevVol dilate(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int
   if (ncols == 0) {
     check(ctx, hipMemsetAsync(out_off, 0, sizeof(int64_t), ctx->stream), "memset");
     out.z = ws(ctx, out_z_slot, 16);
+    out.count = 0;
     return out;
   }
   if (takes_direct(ctx, rint)) {
@@ -889,7 +1008,7 @@ DevVol dilate(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int
       ws(ctx, kG_LISTS, size_t(nt) * 2 * gocap * vo::kWave * sizeof(double));
     }
     const vo::InputCheck<T> c{in.off, static_cast<const T*>(in.z), chk_range, chk_lo, chk_hi};
-    if (dilate_direct<T>(ctx, in, R, ax, c, chk_word, out_off, out_z_slot, out, t1, t2)) return out;
+    if (dilate_direct<T>(ctx, in, R, ax, c, chk_word, out_off, out_z_slot, out, t1, t2, by_rule)) return out;
   }
   std::vector<double> htab_host;  // outlives the uploads (the gather is followed by a synchronisation)
   int chunk1 = std::min(Shapes<T>::p1_cmax, 32);
@@ -1115,6 +1234,22 @@ DevVol dilate(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int
   return out;
 }
 
+// The form is chosen by the volume; what the sweeps then refuse for want of
+// capacity (columns of very many segments) the one-pass form may still take.
+template <class T>
+DevVol dilate(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int out_z_slot, double* t1, double* t2) {
+  const auto fused = ctx->fused;
+  bool by_rule = false;
+  try {
+    return dilate_as<T>(ctx, in, R, out_off_slot, out_z_slot, t1, t2, &by_rule);
+  } catch (const Failure& f) {
+    if (f.code != VO_ERR_CAPACITY || !by_rule) throw;
+  }
+  ctx->error.clear();
+  ctx->fused = fused;
+  return dilate_as<T>(ctx, in, R, out_off_slot, out_z_slot, t1, t2, nullptr);
+}
+
 // Device-side input check of the resident volumes of this call (device
 // entry points; the host-buffer entry point checks on the host).  Nothing
 // waits for it here: the result is copied to host_words[3] and looked at by
@@ -1232,7 +1367,6 @@ DevVol column_transform(vo_context* ctx, bool ring, const DevVol& in, T lo, T hi
     out.ny = ony;
     out.off = off;
     out.z = z;
-    out.count = -1;
     out.outer = ring;
     out.pending = !ring;
     return out;
@@ -1450,7 +1584,6 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
     vol[j].ny = jb.in.ny;
     vol[j].off = jb.in.offsets;
     vol[j].z = jb.in.z;
-    vol[j].count = -1;
   }
   if (t1) *t1 = 0;
   if (t2) *t2 = 0;
@@ -2083,7 +2216,6 @@ void autotune(vo_context* ctx, const vo_volume* sample, int n, const double* rad
   in.ny = sample->ny;
   in.off = sample->offsets;
   in.z = sample->z;
-  in.count = -1;
   const int forced = ctx->zsweep_events;
   struct Sweeps {  // the shapes it tunes are the two sweeps'
     vo_context* c;
@@ -2702,7 +2834,6 @@ int vo_morph_device(vo_context* ctx, int op, int precision, double radius, const
     v.ny = in->ny;
     v.off = in->offsets;
     v.z = in->z;
-    v.count = -1;
     DevVol r = v;
     if (op == VO_OP_NOOP) {
       const int64_t n = int64_t(in->nx) * in->ny;

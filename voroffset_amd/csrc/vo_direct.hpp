@@ -693,7 +693,7 @@ __device__ void direct_tile(const DirectArgs<T>& g, int tile, int64_t slot, Dire
   // With kSplit > 1 a wavefront takes its share of the own block's columns
   // (the first stage's are everyone's: without that cover the others' segments
   // would all stay) and of the other blocks.
-  const bool mine = kSplit == 1 || ((lx >> 1) + (ly >> 1) * (kSplit == 8 ? 5 : 1)) % kSplit == part;
+  const bool mine = kSplit == 1 || ((lx >> 1) + (ly >> 1)) % kSplit == part;
   const int first_mask = rint >= 12 ? 3 : (rint >= 4 ? 1 : 0), first_at = rint >= 12 ? 2 : 0;
   for (int g0 = 0; g0 < g.norder; g0 += kWave) {
     // 64 blocks at a time, one lane each: their summaries
@@ -863,13 +863,14 @@ constexpr int direct_waves() {
 }
 
 // One tile per workgroup of kSplit wavefronts.  Where only the device knows
-// how many endpoints the volume has, two launches of different splits go out
-// and the one whose range does not hold them returns at once (its 4,600 empty
-// workgroups cost 4-7 us at 544^2; reading the count back would cost a wait).
+// how many endpoints the volume has, and nothing else depends on them, two
+// launches of different splits go out and the one whose range does not hold
+// them returns at once (its 4,600 empty workgroups cost 4-7 us at 544^2; a
+// first call that waits for the answer instead 60).
 template <class T, int kList, bool kLdsTable, int kSplit>
 __global__ __launch_bounds__(kWave* kSplit, (direct_waves<kList, kSplit>())) void direct_kernel(DirectArgs<T> g) {
   __shared__ DirectSmem<T, kList> sm[kSplit];
-  const int64_t endpoints = g.off[int64_t(g.nx) * g.ny];
+  const int64_t ncols = int64_t(g.nx) * g.ny, endpoints = g.off[ncols] - g.off[0];
   if (endpoints < g.least || endpoints > g.most) return;
   const double* htab = stage_htab<kLdsTable>(g.htab, g.rint);
   const int64_t i = xcd_tile(blockIdx.x, gridDim.x);

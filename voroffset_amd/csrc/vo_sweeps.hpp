@@ -744,8 +744,13 @@ __global__ __launch_bounds__(kWave) void pass2_kernel(Pass2Args<T> g) {
 
 // The dilation's control words cleared in one launch before pass 1: the
 // status, the count of tiles the gather gives back, and the element past the
-// output lengths (so that their exclusive scan ends with the total).
-__global__ void reset_words_kernel(int* status, int* tiles, int64_t* len_end, int* check_word) {
+// output lengths (so that their exclusive scan ends with the total).  Where
+// `host_count` is given (pinned), it gets the endpoints of the volume whose
+// columns end at off[ncols], which the host waits for.
+__global__ void reset_words_kernel(int* status, int* tiles, int64_t* len_end, int* check_word, const int64_t* off = nullptr,
+                                   int64_t ncols = 0, int64_t* host_count = nullptr) {
+  if (host_count)
+    __hip_atomic_store(host_count, max(off[ncols] - off[0], int64_t(0)), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   *status = 0;
   *tiles = 0;
   *len_end = 0;
