@@ -159,6 +159,11 @@ int vo_copy_device(vo_context* ctx, int n, void* const* dst, const void* const* 
  * (a tuning signal).  No reference counterpart. */
 int vo_last_batch_alone(const vo_context* ctx, int* jobs);
 
+/* Intervals per column the next batch on `ctx` reserves room for (24; 48 once
+ * a volume of a batch outgrew that): with it a caller can tell the memory a
+ * batch will take.  No reference counterpart. */
+int vo_list_capacity(const vo_context* ctx, int* intervals);
+
 /* Parity metrics on a device volume (z of the given precision): the measure
  * spacing^3 * sum of segment lengths and the number of segments, as
  * CompressedVolume::get_volume / numSegments (src/vor3d/CompressedVolume.cpp:61-83;

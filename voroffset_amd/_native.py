@@ -32,7 +32,8 @@ EXPORTS = ("vo_create", "vo_destroy", "vo_last_error", "vo_morph", "vo_result_sh
            "vo_result_free", "vo_morph_device", "vo_last_stats", "vo_rasterize", "vo_morph_batch_device",
            "vo_last_batch_alone", "vo_measure_device", "vo_xor_device",
            "vo_dexel_mesh", "vo_mesh_shape", "vo_mesh_copy", "vo_mesh_free", "vo_autotune", "vo_tuning_save",
-           "vo_tuning_load", "vo_tuning_get", "vo_pass1", "vo_triples_shape", "vo_triples_copy", "vo_triples_free", "vo_copy_device", "vo_morph_device_noalloc")
+           "vo_tuning_load", "vo_tuning_get", "vo_pass1", "vo_triples_shape", "vo_triples_copy", "vo_triples_free", "vo_copy_device", "vo_morph_device_noalloc",
+           "vo_list_capacity")
 
 
 class VoError(RuntimeError):
@@ -124,6 +125,8 @@ def lib():
         L.vo_copy_device.restype = i32
         L.vo_last_batch_alone.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
         L.vo_last_batch_alone.restype = i32
+        L.vo_list_capacity.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
+        L.vo_list_capacity.restype = i32
         _lib = L
     return _lib
 
@@ -349,6 +352,12 @@ class Context:
         """Jobs of the last batch that were redone by the single-volume path."""
         n = ctypes.c_int(0)
         lib().vo_last_batch_alone(self._h, ctypes.byref(n))
+        return n.value
+
+    def list_capacity(self):
+        """Intervals per column the next batch reserves room for."""
+        n = ctypes.c_int(0)
+        lib().vo_list_capacity(self._h, ctypes.byref(n))
         return n.value
 
     def last_stats(self):

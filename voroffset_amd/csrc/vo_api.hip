@@ -140,6 +140,7 @@ inline bool rules_count(double R) { return R < 6; }
 // Entries of a lane's interval list kept in LDS: the long list where columns
 // keep several intervals (small radii) or LDS does not decide how many waves
 // fit (split tiles), the short one elsewhere.
+constexpr int kListRoom = 24, kListRoomMost = 64;  // intervals a list starts with room for, and is kept at
 constexpr int kDirectListLong = 8, kDirectListShort = 3, kDirectSmallR = 3;
 inline int direct_list(int rint, int split) {
   return split > 1 || rint <= kDirectSmallR ? kDirectListLong : kDirectListShort;
@@ -288,7 +289,9 @@ struct vo_context {
   int dtab_norder = 0;
   bool two_pass = false;  // VO_PASS1=zsweep, vo_pass1, vo_autotune: keep to the two sweeps
   bool asked_sweeps = false;  // what the last device-held volume whose size was asked for took
-  int direct_cap = 24;    // intervals per list of the one-pass form (grows on overflow)
+  // intervals per list of the one-pass form, of single volumes and of batches
+  // (whose memory it decides, see vo_list_capacity); each grows on overflow
+  int direct_cap = kListRoom, batch_cap = kListRoom;
   bool chain_dirty = false;  // a call failed: the chained scan's words may not be zero
   int64_t spec_out = 0;  // endpoints the next dilation's output is first sized for
   // an input check left to the pass 1 of the operation's first dilation
@@ -929,9 +932,11 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
     a.cap = c2;
     a.garena = int64_t(2) * c2 * vo::kWave;
     a.spill = static_cast<double*>(ws(ctx, kG_LISTS, list_bytes(nfall, c2)));
-    if (c2 <= 64) ctx->direct_cap = c2;  // the next calls start with the room this one needed
     todo = nfall;
   }
+  // the next calls start with the room this one needed
+  if (!ctx->arena.on)
+    while (ctx->direct_cap < a.cap && 2 * ctx->direct_cap <= kListRoomMost) ctx->direct_cap *= 2;
   ctx->last_fallback_tiles = 0;
   if (t1 || t2) {
     float ms1 = 0, ms2 = 0;
@@ -1638,7 +1643,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   int ocap = 0;
   for (int j = 0; j < n; ++j)
     if (inprog[j] && op[j] != VO_OP_NOOP)
-      ocap = std::max(ocap, direct ? ctx->direct_cap : ocap_for(ctx, int(std::floor(R[j]))));
+      ocap = std::max(ocap, direct ? ctx->batch_cap : ocap_for(ctx, int(std::floor(R[j]))));
   struct Cur {
     int nx, ny;
     int64_t E;
@@ -2047,6 +2052,9 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
     out[j].z_hi = zhi[j];
     if (out_count) out_count[j] = count[k];
   }
+  bool overflowed = false;
+  for (int j = 0; j < n; ++j) overflowed = overflowed || (inprog[j] && st_host[j] != 0);
+  if (direct && overflowed && 2 * ctx->batch_cap <= kListRoomMost) ctx->batch_cap *= 2;  // from the next batch on
   for (int j = 0; j < n; ++j) {
     if (inprog[j] && st_host[j] == 0) continue;
     if (op[j] == VO_OP_NOOP) {
@@ -2982,6 +2990,12 @@ int vo_tuning_load(vo_context* ctx, const char* path) {
 int vo_last_batch_alone(const vo_context* ctx, int* jobs) {
   if (!ctx || !jobs) return VO_ERR_ARGUMENT;
   *jobs = ctx->last_batch_alone;
+  return VO_OK;
+}
+
+int vo_list_capacity(const vo_context* ctx, int* intervals) {
+  if (!ctx || !intervals) return VO_ERR_ARGUMENT;
+  *intervals = ctx->batch_cap;
   return VO_OK;
 }
 

@@ -21,7 +21,9 @@ import numpy as np
 from . import _native
 
 OPS = ("dilation", "erosion", "closing", "opening", "noop")
-_DILATIONS = {"noop": 0, "dilation": 1, "erosion": 1, "closing": 2, "opening": 2}
+_STEPS = {"noop": (), "dilation": ("dilate",), "erosion": ("ring", "dilate", "crop"),
+          "closing": ("dilate", "ring", "dilate", "crop"), "opening": ("ring", "dilate", "crop", "dilate")}
+_DILATIONS = {op: steps.count("dilate") for op, steps in _STEPS.items()}
 
 
 @dataclasses.dataclass
@@ -87,28 +89,30 @@ class Request:
 
 
 def footprint_bytes(ncols, endpoints, op, storage_bytes=4, caps=96, ocap=24):
-    """Estimated device bytes a job occupies inside a batch, per column: the
-    pass-1 slots (lo, hi and a 16-bit line offset per slot), their block
-    summaries (lo and hi per 8 slots) and last hi, the triple count, the
-    gather's interval lists (2 * ocap doubles whatever the storage), its
-    output arena (2 * ocap endpoints), the start, length and offset words;
-    plus the outputs of the job's stages at their bounds (the batch program
-    sizes them before it runs).  ocap is the largest list capacity a batch uses (24 when
-    it holds a radius below 6, 16 otherwise).  An upper bound: jobs with radii
-    below 256 run in one pass and keep no pass-1 slots."""
+    """Estimated device bytes a job occupies inside a batch.  Per column, what
+    the larger of the two forms keeps: the two sweeps their pass-1 slots (lo,
+    hi and a 16-bit line offset per slot), the slots' block summaries (lo and
+    hi per 8 slots), the last hi, the triple count and the gather's interval
+    lists (2 * ocap doubles whatever the storage); the one pass (radii below
+    256) the columns' ends and starts and its lists past their LDS entries (at
+    most 4 * (ocap - 8) doubles).  Both: the output arena (2 * ocap endpoints),
+    the start, length and offset words.  Plus the outputs of the job's stages at
+    their bounds, which the batch program sizes before it runs; all of it a
+    quarter larger, as the context allocates.  ocap is the list capacity of the
+    batch (Context.list_capacity)."""
     if op not in _DILATIONS:
         raise ValueError(f"unknown operation {op!r}")
     if _DILATIONS[op] == 0:
         return 0
-    per_col = (caps * (2 * storage_bytes + 2) + 2 * (caps // 8) * storage_bytes + storage_bytes + 4
-               + 2 * ocap * 8 + 2 * ocap * storage_bytes + 8 + 8 + 8)
-    dilations = _DILATIONS[op]
-    complements = {"dilation": 0, "erosion": 2, "closing": 2, "opening": 2}[op]
+    sweeps = caps * (2 * storage_bytes + 2) + 2 * (caps // 8) * storage_bytes + storage_bytes + 4 + 2 * ocap * 8
+    one_pass = 5 * storage_bytes + 8 + max(2 * (ocap - 3), 4 * (ocap - 8)) * 8
+    total = ncols * (max(sweeps, one_pass) + 2 * ocap * storage_bytes + 8 + 8 + 8)
     # stage outputs, each sized for its bound: a dilation's column holds at
     # most ocap intervals, a complement adds at most two endpoints a column
-    volume = (ncols + 1) * 8 + (endpoints + 2 * ncols) * storage_bytes
-    dilated = (ncols + 1) * 8 + 2 * ocap * ncols * storage_bytes
-    return ncols * per_col + dilations * dilated + complements * volume
+    for step in _STEPS[op]:
+        endpoints = 2 * ocap * ncols if step == "dilate" else endpoints + 2 * ncols
+        total += (ncols + 1) * 8 + endpoints * storage_bytes
+    return total + total // 4
 
 
 class MorphoServer:
@@ -172,7 +176,8 @@ class MorphoServer:
 
     def footprint(self, req):
         r = self.vols[req.handle]
-        return footprint_bytes(r.ncols, r.endpoints, req.op, 4 if self.precision == "fp32" else 8)
+        room = getattr(self.ctx, "list_capacity", lambda: 24)()
+        return footprint_bytes(r.ncols, r.endpoints, req.op, 4 if self.precision == "fp32" else 8, ocap=room)
 
     def admit(self, now=None):
         """Requests to run next: FIFO while the batch fits the budget (the
