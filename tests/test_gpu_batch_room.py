@@ -1,12 +1,13 @@
 """Batches whose lists outgrow their room: the volumes are redone alone, the
 next batch reserves more, and the estimate that admits jobs knows it; a single
-volume redone with more room, or given up, leaves batches as they are."""
+volume redone with more room, or given up, leaves batches as they are.  And
+batches of few tiles, which two wavefronts share, and of many, one each."""
 
 import numpy as np
 import pytest
 import torch
 
-from voroffset_amd import _native, serve
+from voroffset_amd import _native, serve, synth
 from voroffset_amd.volume import CompressedVolume
 
 pytestmark = pytest.mark.gpu
@@ -87,5 +88,20 @@ def test_single_volumes_leave_batches_alone():
             off, _, _ = ctx.morph_host("dilation", "fp64", 3.0, 9, 9, vol.off, vol.z, zlo, zhi)
             assert np.diff(off).max() == 2 * n
         assert ctx.list_capacity() == 24
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("volumes,side", [(3, 40), (6, 128), (7, 128), (4, 300)])
+def test_shared_tiles(prec, volumes, side):
+    """A launch of up to 1536 (FP64 1024) tiles has two wavefronts a tile."""
+    ctx = _native.Context(0)
+    try:
+        for radii in ((2.0, 3.5), (4.0, 9.0), (10.0, 24.0)):
+            items = [(synth.OPS[k % 4], synth.poisson_columns(side, side - k, lam=2.0 + k, zmax=400, seed=k, z_margin=30),
+                      radii[0] + (radii[1] - radii[0]) * k / volumes) for k in range(volumes)]
+            batch = Batch(items, prec)
+            assert equal(batch.run(ctx), batch.alone(ctx))
     finally:
         ctx.close()

@@ -126,12 +126,13 @@ inline bool prefers_sweeps(const Load& v, double R) {
 // at R = 5 892 -> 776).  Past 3072 tiles that gain begins at R = 5, at R = 4 for the
 // sparsest (kernel: 512^2 solids closed at R = 4 456 -> 525, tubes as above), before
 // them at R = 3 (300^2 tubes 180 -> 153; closed at R = 1 149 -> 166).
+constexpr int64_t kPaired(bool wide) { return wide ? 1024 : 1536; }
 inline int direct_split(const Load& v, double R) {
   const int64_t n = v.ntiles;
   const bool dense = v.endpoints > v.sparse();
   if (R < 4 && v.above(R < 1 ? 16 : (R < 2 ? 48 : (R < 3 ? 20 : 100)))) return 1;
   if (n <= kSharedTiles) return R < 4 && dense ? 2 : 4;
-  if (n <= (v.wide ? 1024 : 1536)) return R < 64 && (R >= 6 || !v.above(48)) ? 2 : 1;
+  if (n <= kPaired(v.wide)) return R < 64 && (R >= 6 || !v.above(48)) ? 2 : 1;
   if (R < 3 || R >= 16 || n > kPairedSparseTiles || dense) return 1;
   return n <= kPairedMidTiles || R >= 5 || (R >= 4 && !v.outer && !v.above(1.5)) ? 2 : 1;
 }
@@ -646,28 +647,47 @@ struct DirectTable {
   std::vector<int2> order;
 };
 
+// Distance between the nearest columns of two blocks `d` blocks apart.
+int block_gap(int d) { return d == 0 ? 0 : vo::kSide * (std::abs(d) - 1) + 1; }
+
+// The blocks in reach of the largest radius, nearest first.  Which of them a
+// smaller radius reaches does not change their order, and sorting them for
+// every job of a batch took time (200 jobs of 24^2 at R = 20: 815 -> 740 us a
+// call).
+const std::vector<int2>& blocks_by_distance() {
+  static const std::vector<int2> all = [] {
+    std::vector<int2> v;
+    const int m = (vo::kDirectMaxR + vo::kSide - 1) / vo::kSide;
+    for (int y = -m; y <= m; ++y)
+      for (int x = -m; x <= m; ++x) v.push_back(int2{x, y});
+    std::stable_sort(v.begin(), v.end(), [](const int2& a, const int2& b) {
+      auto key = [](const int2& o) {
+        return std::make_pair(block_gap(o.x) * block_gap(o.x) + block_gap(o.y) * block_gap(o.y), o.x * o.x + o.y * o.y);
+      };
+      return key(a) < key(b);
+    });
+    return v;
+  }();
+  return all;
+}
+
 DirectTable direct_table(double R, bool along_x) {
   const int rint = int(std::floor(R)), W = vo::direct_htab_width(rint);
   const double R2 = R * R;
   DirectTable t;
-  t.h.resize(size_t(W) * W, std::nan(""));
+  t.h.assign(size_t(W) * W, std::nan(""));
   for (int ax = 0; ax <= rint; ++ax)
     for (int ay = 0; ay <= rint; ++ay) {
       const double dy = along_x ? ax : ay, ad = along_x ? ay : ax;
       const double v = R2 - dy * dy - ad * ad;
-      if (v >= 0) t.h[size_t(ax) * W + ay] = std::sqrt(v);
+      if (v < 0) break;
+      t.h[size_t(ax) * W + ay] = std::sqrt(v);
     }
-  auto gap = [](int d) { return d == 0 ? 0 : vo::kSide * (std::abs(d) - 1) + 1; };
-  const int m = (rint + vo::kSide - 1) / vo::kSide;
-  for (int y = -m; y <= m; ++y)
-    for (int x = -m; x <= m; ++x)
-      if (gap(x) <= rint && gap(y) <= rint && !std::isnan(t.h[size_t(gap(x)) * W + gap(y)])) t.order.push_back(int2{x, y});
-  std::stable_sort(t.order.begin(), t.order.end(), [&](const int2& a, const int2& b) {
-    auto key = [&](const int2& o) {
-      return std::make_pair(gap(o.x) * gap(o.x) + gap(o.y) * gap(o.y), o.x * o.x + o.y * o.y);
-    };
-    return key(a) < key(b);
-  });
+  for (const int2& o : blocks_by_distance()) {
+    const int x = block_gap(o.x), y = block_gap(o.y);
+    if (int64_t(x) * x + int64_t(y) * y > int64_t(rint + 1) * (rint + 1)) break;
+    if (x <= rint && y <= rint && !std::isnan(t.h[size_t(x) * W + y])) t.order.push_back(o);
+  }
   return t;
 }
 
@@ -700,6 +720,16 @@ void launch_direct(vo_context* ctx, int rint, int split, const vo::DirectArgs<T>
     launch(vo::direct_kernel<T, kDirectListShort, false, 1>);
 }
 
+// Wavefronts that share a tile in a batched launch of n tiles (one radius class
+// of one stage; the line is direct_split's.  29 volumes of 48^2 to 101^2 at R = 2
+// to 8: 1549 -> 1369 us; 9 of 48^2 to 173^2, FP64, R = 2 to 5.6: 1549 -> 1327; the
+// two sweeps 1572 and 1280).
+int batch_split(int64_t n, bool wide) { return n <= kPaired(wide) ? 2 : 1; }
+// Doubles of a batched tile's lists past their LDS entries, for either split.
+int64_t batch_list_room(int cap) {
+  return 2 * int64_t(std::max(cap - kDirectListShort, 2 * (cap - kDirectListLong))) * vo::kWave;
+}
+
 // Radius class of a batched job in the one-pass form: the kernel it takes.
 int direct_class(int rint) { return rint <= kDirectSmallR ? 0 : (rint <= vo::kDirectLdsTableMax ? 1 : 2); }
 
@@ -709,15 +739,21 @@ template <class T>
 void launch_direct_batch(vo_context* ctx, int c, int max_rint, const vo::DirectArgs<T>* jobs, const int64_t* tile_base,
                          int njobs, int64_t t0, int64_t n) {
   const int W = vo::direct_htab_width(max_rint);
+  const int split = batch_split(n, sizeof(T) == 8);
+  const size_t table = size_t(W) * W * sizeof(double);
   auto launch = [&](auto kernel, size_t lds) {
-    hipLaunchKernelGGL(kernel, dim3(unsigned(n)), dim3(vo::kWave), lds, ctx->stream, jobs, tile_base, njobs, t0, n);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(n)), dim3(vo::kWave * split), lds, ctx->stream, jobs, tile_base, njobs, t0, n);
   };
-  if (c == 0)
-    launch(vo::direct_batch_kernel<T, kDirectListLong, true>, size_t(W) * W * sizeof(double));
+  if (split == 2 && c < 2)
+    launch(vo::direct_batch_kernel<T, kDirectListLong, true, 2>, table);
+  else if (split == 2)
+    launch(vo::direct_batch_kernel<T, kDirectListLong, false, 2>, 0);
+  else if (c == 0)
+    launch(vo::direct_batch_kernel<T, kDirectListLong, true, 1>, table);
   else if (c == 1)
-    launch(vo::direct_batch_kernel<T, kDirectListShort, true>, size_t(W) * W * sizeof(double));
+    launch(vo::direct_batch_kernel<T, kDirectListShort, true, 1>, table);
   else
-    launch(vo::direct_batch_kernel<T, kDirectListShort, false>, 0);
+    launch(vo::direct_batch_kernel<T, kDirectListShort, false, 1>, 0);
 }
 
 // One dilation in one pass (vo_direct.hpp): returns false, with nothing done,
@@ -1705,7 +1741,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   // 3. workspace, sized for the largest step (steps run one after the other)
   const int caps = ctx->p1_caps;
   const int64_t garena = int64_t(vo::kGatherTile) * 2 * ocap;
-  const int64_t list_tile = 2 * int64_t(direct ? ocap - kDirectListShort : ocap) * vo::kWave;
+  const int64_t list_tile = direct ? batch_list_room(ocap) : 2 * int64_t(ocap) * vo::kWave;
   for (auto& st : steps) {
     st.off = static_cast<int64_t*>(ws(ctx, st.off_slot, size_t(st.C + 1) * sizeof(int64_t)));
     st.z = ws(ctx, st.z_slot, size_t(std::max<int64_t>(st.zcap, 1)) * sizeof(T));

@@ -880,18 +880,19 @@ __global__ __launch_bounds__(kWave* kSplit, (direct_waves<kList, kSplit>())) voi
 }
 
 // Batched: job j owns the global tiles [tile_base[j], tile_base[j + 1]); this
-// launch covers the n tiles from t0 on (one radius class).
-template <class T, int kList, bool kLdsTable>
-__global__ __launch_bounds__(kWave, (direct_waves<kList, 1>())) void direct_batch_kernel(const DirectArgs<T>* jobs,
-                                                                                    const int64_t* tile_base, int njobs,
-                                                                                    int64_t t0, int64_t n) {
-  __shared__ DirectSmem<T, kList> sm[1];
+// launch covers the n tiles from t0 on (one radius class), kSplit wavefronts
+// each.
+template <class T, int kList, bool kLdsTable, int kSplit>
+__global__ __launch_bounds__(kWave* kSplit, (direct_waves<kList, kSplit>())) void direct_batch_kernel(
+    const DirectArgs<T>* jobs, const int64_t* tile_base, int njobs, int64_t t0, int64_t n) {
+  __shared__ DirectSmem<T, kList> sm[kSplit];
   const int64_t t = t0 + xcd_chunk_tile(blockIdx.x, n);
   const int j = find_job(tile_base, njobs, t);
   const DirectArgs<T> g = jobs[j];
   const double* htab = stage_htab<kLdsTable>(g.htab, g.rint);
   const int64_t i = t - tile_base[j];
-  direct_tile<T, kList, 1>(g, int(i), i, sm, 0, htab);
+  const int part = kSplit > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;
+  direct_tile<T, kList, kSplit>(g, int(i), i, sm, part, htab);
 }
 
 }  // namespace vo
