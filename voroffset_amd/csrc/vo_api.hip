@@ -295,6 +295,7 @@ struct vo_context {
   int direct_cap = kListRoom, batch_cap = kListRoom;
   bool chain_dirty = false;  // a call failed: the chained scan's words may not be zero
   int64_t spec_out = 0;  // endpoints the next dilation's output is first sized for
+  const int64_t* counted = nullptr;  // offsets whose volume this call's input check counts, into host_words[7]
   // an input check left to the pass 1 of the operation's first dilation
   // (word == null: none pending); see defer_input_check
   struct {
@@ -472,6 +473,20 @@ int64_t await_count(vo_context* ctx) {
     break;
   }
   return n;
+}
+
+// The endpoints of a volume in device memory, whose offsets may begin anywhere
+// in a buffer it shares with others.  Waits for the stream.
+int64_t read_count(vo_context* ctx, const int64_t* off, int64_t ncols) {
+  if (ctx->counted == off) {  // by this call's input check
+    ctx->counted = nullptr;
+    sync(ctx);
+    return ctx->host_words[7];
+  }
+  hipLaunchKernelGGL(vo::report_count_kernel, dim3(1), dim3(1), 0, ctx->stream, off, ncols, ctx->host_words);
+  check(ctx, hipGetLastError(), "count launch");
+  sync(ctx);
+  return ctx->host_words[0];
 }
 
 std::string status_text(int s) {
@@ -1319,7 +1334,11 @@ void enqueue_input_check(vo_context* ctx, const std::vector<vo::InputCheck<T>>& 
   const int K = int(jobs.size());
   ctx->check_jobs = job_ids;
   int* word = static_cast<int*>(ws(ctx, kV_WORD, 2 * sizeof(int)));
-  hipLaunchKernelGGL(vo::init_check_words_kernel, dim3(1), dim3(1), 0, ctx->stream, word);
+  // (a volume checked alone has its endpoints counted with it)
+  const bool one = K == 1 && ncols[0] > 0;
+  ctx->counted = one ? jobs[0].off : nullptr;
+  hipLaunchKernelGGL(vo::init_check_words_kernel, dim3(1), dim3(1), 0, ctx->stream, word, one ? jobs[0].off : nullptr,
+                     one ? ncols[0] : 0, one ? ctx->host_words + 7 : nullptr);
   check(ctx, hipGetLastError(), "input check words");
   ctx->check_base.assign(size_t(K) + 1, 0);
   for (int k = 0; k < K; ++k) ctx->check_base[k + 1] = ctx->check_base[k] + ncols[k];
@@ -1387,9 +1406,7 @@ DevVol column_transform(vo_context* ctx, bool ring, const DevVol& in, T lo, T hi
     // count there is room for the result before its size is known, and
     // lengths, offsets and data are one launch with nothing to wait for.
     const int64_t in_cols = int64_t(in.nx) * in.ny;
-    // (a volume the caller keeps on the device: its last offset, which is no
-    // less than what its columns hold)
-    const int64_t count = in.count >= 0 ? in.count : (in_cols ? read_word(ctx, in.off + in_cols) : 0);
+    const int64_t count = in.count >= 0 ? in.count : (in_cols ? read_count(ctx, in.off, in_cols) : 0);
     const int64_t cap = count + 2 * n;
     int64_t* off = static_cast<int64_t*>(ws(ctx, off_slot, (n + 1) * sizeof(int64_t)));
     T* z = static_cast<T*>(ws(ctx, z_slot, size_t(std::max<int64_t>(cap, 1)) * sizeof(T)));
@@ -2327,6 +2344,7 @@ int guarded(vo_context* ctx, const std::function<void()>& body) {
   // a call's input check never outlives it
   ctx->check_input = false;
   ctx->fused.word = nullptr;
+  ctx->counted = nullptr;
   (void)hipGetLastError();  // an error left by an earlier, already reported call is not this call's
   try {
     check(ctx, hipSetDevice(ctx->device), "hipSetDevice");

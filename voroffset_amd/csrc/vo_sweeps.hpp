@@ -759,7 +759,12 @@ __global__ void reset_words_kernel(int* status, int* tiles, int64_t* len_end, in
     check_word[1] = 0x7f7f7f7f;
   }
 }
-// ... and reported in one launch to the host's pinned words (device-mapped
+// The endpoints of a volume, to the host's pinned word.
+__global__ void report_count_kernel(const int64_t* off, int64_t ncols, int64_t* host) {
+  *host = off[ncols] - off[0];
+  __threadfence_system();
+}
+// The control words reported in one launch to the host's pinned words (device-mapped
 // memory, read after the stream is synchronised): [0] the output total,
 // [1] the status, [2] the tiles given back, [3] the input check's two words
 // when pass 1 did the check.
@@ -773,9 +778,14 @@ __global__ void report_words_kernel(const int64_t* total, const int* status, con
 }
 // The input check's words before its kernel: no failure yet, and the
 // largest job index (atomicMin keeps the smallest failing one).
-__global__ void init_check_words_kernel(int* word) {
+// (and, where asked for, the endpoints of the volume, to the host's pinned word)
+__global__ void init_check_words_kernel(int* word, const int64_t* off = nullptr, int64_t ncols = 0, int64_t* host = nullptr) {
   word[0] = 0;
   word[1] = 0x7f7f7f7f;
+  if (host) {
+    *host = off[ncols] - off[0];
+    __threadfence_system();
+  }
 }
 
 // Gather per-column results (start, count) into CSR at precomputed offsets.
