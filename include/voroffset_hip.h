@@ -13,7 +13,7 @@
  *
  * Conventions (mirroring the reference):
  *   - radius is in dexels; time_1 / time_2 report pass 1 / pass 2 in ms (in
- *     the one-pass form, radii below 256: its block summaries / the dilation);
+ *     the one-pass form: its block summaries / the dilation);
  *   - erosion complements on a grid grown by one ring of full columns over
  *     [z_lo - 1, z_hi + 1], dilates, crops and complements within [z_lo, z_hi],
  *     where z_lo = origin_z / spacing and z_hi = z_lo + 2*padding + extent_z / spacing;
@@ -196,9 +196,10 @@ void vo_mesh_free(vo_mesh_result* r);
  * list capacity (8, 16, 24, 32) on `sample` (a device volume of the given
  * precision), `reps` runs each, and keeps the fastest per radius bucket
  * ([0,8), [8,16), [16,32), [32,64), [64,128)) in `ctx`; results do not
- * depend on the choice.  It times and tunes the two-sweep form; a dilation in
- * one pass (radii below 256, unless VO_PASS1 names a form) has nothing to
- * tune.  The table can be saved, loaded and read back. */
+ * depend on the choice.  It times and tunes the two sweeps, which radii from 256
+ * take, below radius 6 volumes they are faster on (dense columns, tiny or very
+ * thin grids), and contexts for which VO_PASS1 names a form; a dilation in one
+ * pass has nothing to tune.  The table can be saved, loaded and read back. */
 int vo_autotune(vo_context* ctx, int precision, const vo_volume* sample, int num_radii, const double* radii,
                 int reps);
 int vo_tuning_save(const vo_context* ctx, const char* path);
@@ -220,9 +221,11 @@ int vo_rasterize(vo_context* ctx, const double* vertices, int64_t num_vertices, 
                  vo_result** out);
 
 /* Statistics of the last dilation on `ctx`: the number of output endpoints
- * and the number of 64-column pass-2 tiles whose interval lists outgrew LDS
- * and were recomputed by the sweep form (a tuning signal; results do not
- * depend on it).  No reference counterpart. */
+ * and the number of tiles whose interval lists outgrew their room and were
+ * computed again: in the one-pass form tiles of 8 x 8 columns, with twice the
+ * room (counted each time), in the two sweeps pass-2 tiles of 64 columns, by
+ * the sweep form (a tuning signal; results do not depend on it).  No reference
+ * counterpart. */
 int vo_last_stats(const vo_context* ctx, int64_t* output_endpoints, int64_t* fallback_tiles);
 
 #ifdef __cplusplus

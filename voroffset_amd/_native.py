@@ -361,7 +361,7 @@ class Context:
         return n.value
 
     def last_stats(self):
-        """(output endpoints, pass-2 tiles recomputed by the sweep form) of the last dilation."""
+        """(output endpoints, tiles computed again) of the last dilation."""
         a, b = ctypes.c_int64(), ctypes.c_int64()
         lib().vo_last_stats(self._h, ctypes.byref(a), ctypes.byref(b))
         return a.value, b.value

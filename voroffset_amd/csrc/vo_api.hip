@@ -280,7 +280,7 @@ struct vo_context {
   bool batch_queue = false;       // VO_BATCH_QUEUE=1: persistent work-queue grids for the batched passes
   int num_cus = 0;                // compute units of the device
   std::map<std::pair<const void*, size_t>, int> resident;  // workgroups per CU, by kernel and dynamic LDS
-  int last_fallback_tiles = 0;
+  int last_fallback_tiles = 0;    // tiles of the last dilation that were computed again
   // the radius whose gather table the H-table slot holds (-1: none; a call
   // with the same radius skips the upload)
   double htab_R = -1;
@@ -907,6 +907,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
                       o_z, int64_t(2) * cap * vo::kWave, 0, o_start, o_len, cap, spill, tiles, status, nullptr};
   int64_t todo = ntiles, done_tiles = 0;  // tiles of this launch, and output regions used by earlier ones
   int64_t total = -1;
+  int redone = 0;
   bool copied = false;
   for (;;) {
     if (sparse_split != split) {
@@ -952,6 +953,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
     // (their output goes past the earlier ones'), up to kGatherRoomBytes
     if (ctx->arena.on) return false;
     done_tiles += todo * a.cap;
+    redone += int(nfall);
     const int c2 = 2 * a.cap;
     const size_t room = size_t(done_tiles + nfall * c2) * 2 * vo::kWave * sizeof(T) + list_bytes(nfall, c2);
     if (room > kGatherRoomBytes || c2 > vo::kDirectMaxList) return false;
@@ -988,7 +990,7 @@ bool dilate_direct(vo_context* ctx, const DevVol& in, double R, const Axis& ax, 
   // the next calls start with the room this one needed
   if (!ctx->arena.on)
     while (ctx->direct_cap < a.cap && 2 * ctx->direct_cap <= kListRoomMost) ctx->direct_cap *= 2;
-  ctx->last_fallback_tiles = 0;
+  ctx->last_fallback_tiles = redone;
   if (t1 || t2) {
     float ms1 = 0, ms2 = 0;
     check(ctx, hipEventElapsedTime(&ms1, ctx->ev[0], ctx->ev[1]), "elapsed");
