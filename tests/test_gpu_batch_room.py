@@ -95,7 +95,7 @@ def test_single_volumes_leave_batches_alone():
 @pytest.mark.parametrize("prec", ["fp32", "fp64"])
 @pytest.mark.parametrize("volumes,side", [(3, 40), (6, 128), (7, 128), (4, 300)])
 def test_shared_tiles(prec, volumes, side):
-    """A launch of up to 1536 (FP64 1024) tiles has two wavefronts a tile."""
+    """A launch of up to 1280 (FP64 1024) tiles has two wavefronts a tile."""
     ctx = _native.Context(0)
     try:
         for radii in ((2.0, 3.5), (4.0, 9.0), (10.0, 24.0)):

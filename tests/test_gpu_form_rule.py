@@ -64,7 +64,8 @@ def test_lines_of_the_rule(contexts, prec, nx, ny, segments, r):
     same(contexts, volume(nx, ny, segments, nx + segments), "dilation", prec, r)
 
 
-@pytest.mark.parametrize("nx,ny", [(384, 256), (385, 256), (768, 256), (769, 256), (1024, 384), (1025, 384)])
+@pytest.mark.parametrize("nx,ny", [(320, 256), (321, 256), (512, 256), (513, 256), (768, 256), (769, 256), (1024, 384),
+                                   (1025, 384)])
 @pytest.mark.parametrize("segments", [0.4, 1.5, 2.5])
 @pytest.mark.parametrize("op,r", [("dilation", 2.0), ("dilation", 3.5), ("dilation", 4.0), ("dilation", 5.0),
                                   ("dilation", 15.9), ("dilation", 16.0), ("closing", 4.0), ("closing", 5.5)])

@@ -5,8 +5,9 @@
 //   summary kernel -> the ends and counts of every column and 8 x 8 block
 //   direct kernel  -> per-column output intervals, in one pass over the input
 //   assemble       -> offsets, CSR result and report in one chained scan
-// Radii of 256 and more, lists past the direct form's room, and the forms
-// VO_PASS1 / VO_PASS2 name take two sweeps instead:
+// Radii of 256 and more, volumes on which they are faster (prefers_sweeps),
+// lists past the direct form's room, and the forms VO_PASS1 / VO_PASS2 name
+// take two sweeps instead:
 //   pass 1 kernel  -> per-column triples (lo, hi, dy) in a chunked arena
 //   pass 2 kernel  -> per-column output intervals in a chunked arena
 //   exclusive scan of the output lengths + gather -> CSR result
@@ -110,30 +111,33 @@ inline bool prefers_sweeps(const Load& v, double R) {
 }
 // Wavefronts that share a tile.  Few tiles leave most of the card idle, each a
 // long serial chain: up to 512 four of them do (86 x 88 solids at R = 6.4: 400
-// -> 191, 212 x 118 closing at R = 27: 466 -> 171), below R = 4 only sparse ones (139 x
-// 121 solids eroded at R = 2.4: 238, with two 282), else two: lists are long and want
-// the whole cover (64^2, e = 12, R = 3: 0.82, 0.76 and 0.92 times the sweeps for one,
-// two and four); those of dense columns are not shared (64^2, e = 80: R = 2 1.3, 3.1 and 3.2; R = 1.5 1.2, 2.3 and
-// 1.9).  Up to as many tiles as are resident together two share one (kernel,
-// 270^2, e = 4: R = 2 180 -> 144, R = 4 191 -> 132, R = 8 123 -> 87; 256^2 at R = 20 0.77-0.98 of
-// one, but R = 100 1.07 and R = 200 1.15; 360^2, 2025
-// tiles, 1.1-1.2; FP64, of which fewer are resident: 280^2, 1225 tiles, R = 2.5 1.2-1.4).
+// -> 191, 212 x 118 closing at R = 27: 466 -> 171), below R = 4 up to 10 endpoints
+// a column (139 x 121 solids eroded at R = 2.4: 238, with two 282), else two:
+// lists are long and want the whole cover (64^2, e = 12, R = 3: 0.82, 0.76 and
+// 0.92 times the sweeps for one, two and four); those of dense columns are not
+// shared (64^2, e = 80: R = 2 1.3, 3.1 and 3.2; R = 1.5 1.2, 2.3 and 1.9).
+// Up to as many tiles as are resident together (five such workgroups' LDS on
+// each of 256 CUs, FP64 four) two share one (kernel, 270^2, e = 4: R = 2 180 ->
+// 144, R = 4 191 -> 132, R = 8 123 -> 87; 256^2 at R = 20 0.77-0.98 of one, but
+// R = 100 1.07 and R = 200 1.15; 360^2, 2025 tiles, 1.1-1.2; 177 x 526, 1518
+// tiles, e = 15, R = 2.8 1.36; FP64, 280^2, 1225 tiles, R = 2.5 1.2-1.4).
 // Above, the wavefronts' weaker covers cost more than they give (kernel, 512^2,
 // e = 2: 1.4-1.6 times), except on the tails that filigree and solids have: for
 // columns of few endpoints (a ring complement has two more, and what the
-// dilation before it parted: four are allowed) and radii from 3 to 16, two up to 6144 tiles
-// (kernel, tubes, R = 4 / 8: 400^2 266 -> 163, 418 -> 256; 512^2 306 -> 282, 526 -> 465; closed
-// at R = 5 892 -> 776).  Past 3072 tiles that gain begins at R = 5, at R = 4 for the
-// sparsest (kernel: 512^2 solids closed at R = 4 456 -> 525, tubes as above), before
-// them at R = 3 (300^2 tubes 180 -> 153; closed at R = 1 149 -> 166).
-constexpr int64_t kPaired(bool wide) { return wide ? 1024 : 1536; }
+// dilation before it parted: four are allowed) and radii below 16, two up to
+// 6144 tiles (kernel, tubes, R = 4 / 8: 400^2 266 -> 163, 418 -> 256; 512^2 306 ->
+// 282, 526 -> 465; closed at R = 5 892 -> 776).  Past 3072 tiles that gain begins
+// at R = 5, at R = 4 for the sparsest (kernel: 512^2 solids closed at R = 4 456 ->
+// 525, tubes as above), before them at R = 3 (300^2 tubes 180 -> 153), up to 2048
+// at R = 2 (closing of 300^2 tubes 231 -> 204, at R = 1 149 -> 166).
+constexpr int64_t kPaired(bool wide) { return wide ? 1024 : 1280; }
 inline int direct_split(const Load& v, double R) {
   const int64_t n = v.ntiles;
   const bool dense = v.endpoints > v.sparse();
   if (R < 4 && v.above(R < 1 ? 16 : (R < 2 ? 48 : (R < 3 ? 20 : 100)))) return 1;
-  if (n <= kSharedTiles) return R < 4 && dense ? 2 : 4;
+  if (n <= kSharedTiles) return R < 4 && v.above(v.outer ? 14 : 10) ? 2 : 4;
   if (n <= kPaired(v.wide)) return R < 64 && (R >= 6 || !v.above(48)) ? 2 : 1;
-  if (R < 3 || R >= 16 || n > kPairedSparseTiles || dense) return 1;
+  if (R < (n <= 2048 ? 2 : 3) || R >= 16 || n > kPairedSparseTiles || dense) return 1;
   return n <= kPairedMidTiles || R >= 5 || (R >= 4 && !v.outer && !v.above(1.5)) ? 2 : 1;
 }
 // Whether the host has to know the endpoints (for the form, and small radii's splits).
@@ -740,9 +744,11 @@ void launch_direct(vo_context* ctx, int rint, int split, const vo::DirectArgs<T>
 // to 8: 1549 -> 1369 us; 9 of 48^2 to 173^2, FP64, R = 2 to 5.6: 1549 -> 1327; the
 // two sweeps 1572 and 1280).
 int batch_split(int64_t n, bool wide) { return n <= kPaired(wide) ? 2 : 1; }
-// Doubles of a batched tile's lists past their LDS entries, for either split.
-int64_t batch_list_room(int cap) {
-  return 2 * int64_t(std::max(cap - kDirectListShort, 2 * (cap - kDirectListLong))) * vo::kWave;
+// Doubles of a batched tile's lists past their LDS entries, where one wavefront
+// has it or (`shared`) two may.
+int64_t batch_list_room(int cap, bool shared) {
+  const int one = cap - kDirectListShort, two = 2 * (cap - kDirectListLong);
+  return 2 * int64_t(shared ? std::max(one, two) : one) * vo::kWave;
 }
 
 // Radius class of a batched job in the one-pass form: the kernel it takes.
@@ -1455,6 +1461,7 @@ DevVol column_transform(vo_context* ctx, bool ring, const DevVol& in, T lo, T hi
   out.off = off;
   out.z = z;
   out.count = total;
+  out.outer = ring;
   return out;
 }
 
@@ -1707,6 +1714,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   for (int j = 0; j < n; ++j) cur[j] = Cur{vol[j].nx, vol[j].ny, E[j]};
   std::vector<ProgStep> steps;
   int64_t maxC = 0, maxDilC = 0, maxNT = 0;
+  bool shared = false;  // some launch's tiles are shared by two wavefronts
   for (int s = 0; s < 4; ++s) {
     for (int kind : {int(kStepRing), int(kStepDilate), int(kStepCrop)}) {
       ProgStep st;
@@ -1752,6 +1760,9 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
       if (kind == kStepDilate) {
         maxDilC = std::max(maxDilC, st.C);
         maxNT = std::max(maxNT, st.NT);
+        int64_t tiles[3] = {0, 0, 0};
+        for (int k = 0; k < K; ++k) tiles[class_of(R[st.jobs[k]])] += st.tile_base[k + 1] - st.tile_base[k];
+        for (int64_t n : tiles) shared = shared || (n > 0 && batch_split(n, sizeof(T) == 8) > 1);
       }
       steps.push_back(std::move(st));
     }
@@ -1760,7 +1771,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   // 3. workspace, sized for the largest step (steps run one after the other)
   const int caps = ctx->p1_caps;
   const int64_t garena = int64_t(vo::kGatherTile) * 2 * ocap;
-  const int64_t list_tile = direct ? batch_list_room(ocap) : 2 * int64_t(ocap) * vo::kWave;
+  const int64_t list_tile = direct ? batch_list_room(ocap, shared) : 2 * int64_t(ocap) * vo::kWave;
   for (auto& st : steps) {
     st.off = static_cast<int64_t*>(ws(ctx, st.off_slot, size_t(st.C + 1) * sizeof(int64_t)));
     st.z = ws(ctx, st.z_slot, size_t(std::max<int64_t>(st.zcap, 1)) * sizeof(T));
