@@ -232,6 +232,12 @@ def run_device(ctx, vol, radius, precision, steps, warmup):
     return dt / steps, p1 / steps, p2 / steps, count
 
 
+def takes_sweeps(radius):
+    """Whether dilations by `radius` may take the two sweeps, whose shapes the
+    autotuner picks (the one-pass form has nothing to tune)."""
+    return bool(os.environ.get("VO_PASS1") or os.environ.get("VO_PASS2")) or radius < 6 or radius >= 256
+
+
 def tune_context(ctx, lam, radii, side=256, seed=7):
     """Untimed: autotunes ctx's shapes for these radii on a side x side
     Poisson(lam) sample volume (FP32 storage)."""
@@ -465,7 +471,7 @@ def main():
     ncols = vol.ncols
     ctx = _native.Context(0)
     tuned = None
-    if not args.no_tune:  # untimed: the autotuner picks the shapes for this radius on the workload itself
+    if not args.no_tune and takes_sweeps(R):  # untimed: the autotuner picks the shapes for this radius on the workload itself
         zlo, zhi = vol.z_range()
         shift = _native.storage_shift(zlo, zhi)
         d_off, d_z = _native.DeviceArray(vol.off), _native.DeviceArray((vol.z - shift).astype(np.float32))
@@ -479,7 +485,7 @@ def main():
     step_s, p1_ms, p2_ms, count = run_device(ctx, vol, R, "fp32", args.steps, args.warmup)
     fallback = ctx.last_stats()[1]
     log(f"fp32: {step_s * 1e3:.3f} ms/step, pass1 {p1_ms:.3f} ms, pass2 {p2_ms:.3f} ms, "
-        f"{fallback} pass-2 tiles recomputed by the sweep form")
+        f"{fallback} tiles computed again")
     plain = None
     if not args.no_fp64:
         f64_s, f64_p1, f64_p2, _ = run_device(ctx, vol, R, "fp64", max(3, args.steps // 4), 1)
@@ -487,15 +493,17 @@ def main():
         plain = {"value": round(ncols / f64_s, 1), "ms_per_step": round(f64_s * 1e3, 4),
                  "pass1_ms": round(f64_p1, 4), "pass2_ms": round(f64_p2, 4)}
 
-    # the batch is tuned on its own uneven volumes (shapes tuned on one
-    # uniform sample made it slower: 39.3 ms against 35.6 ms untuned); the
-    # served leg keeps the default shapes
+    # a batch in the two sweeps is tuned on its own uneven volumes (shapes tuned
+    # on one uniform sample made it slower: 39.3 ms against 35.6 ms untuned);
+    # the served leg keeps the default shapes
     items = []
     batched = None
     if args.batch_volumes > 0:
-        # two untimed batches: the first runs eagerly, the second captures the
-        # program into a HIP graph; the timed ones replay it (steady state)
-        batched, more = batched_leg(args.batch_volumes, max(2, args.steps // 5), 2, tune=not args.no_tune)
+        # untimed batches: the first runs eagerly, the second captures the
+        # program into a HIP graph, and after some more its tables' upload
+        # is at its steady speed (14.3 -> 13.5 ms); the timed ones replay it
+        batched, more = batched_leg(args.batch_volumes, max(2, args.steps // 5), 16,
+                                    tune=not args.no_tune and takes_sweeps(16.0))
         items += more
 
     served = None
@@ -518,13 +526,14 @@ def main():
     s_in = vol.num_segments() / ncols
     s_out = count / 2 / ncols
     roofline = None
-    if R < 256 and not os.environ.get("VO_PASS1"):  # the one-pass form: summaries, then the dilation
+    if not takes_sweeps(R):  # the one-pass form: summaries, then the dilation
         b = ncols * ((2 * s_in * E + 8) + (2 * s_out * E + 8))
         name, ms = "direct", p2_ms
         achieved = b / (ms * 1e-3) / 1e9
         # the instantiation the timed steps ran (FP32 storage, this radius);
         # counters measured on another one are not attached
-        inst = f"direct_kernel<float, {8 if int(R) <= 3 else 3}, {'true' if int(R) <= 9 else 'false'}, 1>"
+        # (one wavefront a tile: the default grid's 16384 tiles)
+        inst = f"direct_kernel<float, 3, {'true' if int(R) <= 9 else 'false'}, 1>"
         traffic, tnote = None, "no counter profile of this kernel in profiles/"
         tpath = os.path.join(ROOT, "profiles", f"traffic_{name}_1024_r16.json")
         if os.path.exists(tpath):
@@ -555,7 +564,7 @@ def main():
                                f"Exp(40) gaps and lengths, dilation r={R:g}, one volume per launch",
                    "grid": [side, side], "radius": R, "storage": "fp32", "op": "dilation",
                    "pass1_ms": round(p1_ms, 4), "pass2_ms": round(p2_ms, 4),
-                   "plain_fp64": plain, "pass2_sweep_tiles": fallback, "autotuned": tuned, "batched": batched,
+                   "plain_fp64": plain, "tiles_computed_again": fallback, "autotuned": tuned, "batched": batched,
                    "served": served,
                    "s_in": round(s_in, 4), "s_out": round(s_out, 4), "m_oracle": m,
                    "precision": precision},
