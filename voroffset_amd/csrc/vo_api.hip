@@ -745,10 +745,9 @@ void launch_direct(vo_context* ctx, int rint, int split, const vo::DirectArgs<T>
 // two sweeps 1572 and 1280).
 int batch_split(int64_t n, bool wide) { return n <= kPaired(wide) ? 2 : 1; }
 // Doubles of a batched tile's lists past their LDS entries, where one wavefront
-// has it or (`shared`) two may.
+// or (`shared`) two have it.
 int64_t batch_list_room(int cap, bool shared) {
-  const int one = cap - kDirectListShort, two = 2 * (cap - kDirectListLong);
-  return 2 * int64_t(shared ? std::max(one, two) : one) * vo::kWave;
+  return 2 * int64_t(shared ? 2 * (cap - kDirectListLong) : cap - kDirectListShort) * vo::kWave;
 }
 
 // Radius class of a batched job in the one-pass form: the kernel it takes.
@@ -1601,6 +1600,7 @@ struct ProgStep {
   int64_t* off = nullptr;  // output CSR over the step's columns (absolute into z)
   void* z = nullptr;
   std::vector<int64_t> sum_base;  // one-pass dilation: the summary kernel's workgroups
+  std::vector<int64_t> list_base; // dilation: doubles of the jobs' lists
   size_t t0 = 0, t1 = 0, t2 = 0, t3 = 0, t4 = 0;  // table offsets in the blob
   int64_t cls_t0[3] = {0, 0, 0}, cls_t1[3] = {0, 0, 0};
   int cls_rmax[3] = {0, 0, 0};
@@ -1713,8 +1713,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   std::vector<Cur> cur(n);
   for (int j = 0; j < n; ++j) cur[j] = Cur{vol[j].nx, vol[j].ny, E[j]};
   std::vector<ProgStep> steps;
-  int64_t maxC = 0, maxDilC = 0, maxNT = 0;
-  bool shared = false;  // some launch's tiles are shared by two wavefronts
+  int64_t maxC = 0, maxDilC = 0, maxNT = 0, maxLists = 0;
   for (int s = 0; s < 4; ++s) {
     for (int kind : {int(kStepRing), int(kStepDilate), int(kStepCrop)}) {
       ProgStep st;
@@ -1762,7 +1761,14 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
         maxNT = std::max(maxNT, st.NT);
         int64_t tiles[3] = {0, 0, 0};
         for (int k = 0; k < K; ++k) tiles[class_of(R[st.jobs[k]])] += st.tile_base[k + 1] - st.tile_base[k];
-        for (int64_t n : tiles) shared = shared || (n > 0 && batch_split(n, sizeof(T) == 8) > 1);
+        // (lists past their LDS entries: more of them where two wavefronts share a tile)
+        st.list_base.assign(K + 1, 0);
+        for (int k = 0; k < K; ++k) {
+          const int64_t nt = st.tile_base[k + 1] - st.tile_base[k];
+          const bool shared = batch_split(tiles[class_of(R[st.jobs[k]])], sizeof(T) == 8) > 1;
+          st.list_base[k + 1] = st.list_base[k] + nt * (direct ? batch_list_room(ocap, shared) : 2 * int64_t(ocap) * vo::kWave);
+        }
+        maxLists = std::max(maxLists, st.list_base[K]);
       }
       steps.push_back(std::move(st));
     }
@@ -1771,7 +1777,6 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
   // 3. workspace, sized for the largest step (steps run one after the other)
   const int caps = ctx->p1_caps;
   const int64_t garena = int64_t(vo::kGatherTile) * 2 * ocap;
-  const int64_t list_tile = direct ? batch_list_room(ocap, shared) : 2 * int64_t(ocap) * vo::kWave;
   for (auto& st : steps) {
     st.off = static_cast<int64_t*>(ws(ctx, st.off_slot, size_t(st.C + 1) * sizeof(int64_t)));
     st.z = ws(ctx, st.z_slot, size_t(std::max<int64_t>(st.zcap, 1)) * sizeof(T));
@@ -1800,7 +1805,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
     d_bcnt = static_cast<int*>(ws(ctx, kD_BCNT, size_t(maxNT) * sizeof(int)));
     o_z = static_cast<T*>(ws(ctx, kO_Z, size_t(maxNT) * garena * sizeof(T)));
     o_start = static_cast<int64_t*>(ws(ctx, kO_START, size_t(maxDilC) * sizeof(int64_t)));
-    lists = static_cast<double*>(ws(ctx, kG_LISTS, size_t(maxNT) * list_tile * sizeof(double)));
+    lists = static_cast<double*>(ws(ctx, kG_LISTS, size_t(maxLists) * sizeof(double)));
   } else if (maxDilC > 0) {
     m_lo = static_cast<T*>(ws(ctx, kM_LO, size_t(maxDilC) * caps * sizeof(T)));
     m_hi = static_cast<T*>(ws(ctx, kM_HI, size_t(maxDilC) * caps * sizeof(T)));
@@ -1811,7 +1816,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
     m_cnt = static_cast<int32_t*>(ws(ctx, kM_CNT, size_t(maxDilC) * sizeof(int32_t)));
     o_z = static_cast<T*>(ws(ctx, kO_Z, size_t(maxNT) * garena * sizeof(T)));
     o_start = static_cast<int64_t*>(ws(ctx, kO_START, size_t(maxDilC) * sizeof(int64_t)));
-    lists = static_cast<double*>(ws(ctx, kG_LISTS, size_t(maxNT) * list_tile * sizeof(double)));
+    lists = static_cast<double*>(ws(ctx, kG_LISTS, size_t(maxLists) * sizeof(double)));
   }
   {  // the scan's temporary storage, for the largest step
     size_t tmp = 0;
@@ -1856,7 +1861,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
         a2[k] = vo::DirectArgs<T>{in.nx, in.ny, nbx, nby, rint, in.off, z, a1[k].col, a1[k].at, a1[k].blk, a1[k].bcnt,
                                   reinterpret_cast<const double*>(hat), reinterpret_cast<const int2*>(oat),
                                   int(t.order.size()), o_z, garena, tb * garena, o_start + cb, len + cb, ocap,
-                                  lists + tb * list_tile, nullptr, status + j, nullptr};
+                                  lists + st.list_base[k], nullptr, status + j, nullptr};
         if (st.cls_t1[c] == 0) st.cls_t0[c] = st.tile_base[k];
         st.cls_t1[c] = st.tile_base[k + 1];
         st.cls_rmax[c] = std::max(st.cls_rmax[c], rint);
@@ -1897,7 +1902,7 @@ void morph_batch_device(vo_context* ctx, int n, const vo_job* jobs, vo_volume* o
         a2[k] = vo::Pass2GArgs<T>{ax.nx, ax.ny, rint, R[j] * R[j], m_lo + sb, m_hi + sb, m_dy + sb, caps,
                                   m_cnt + cb, o_z, garena, o_start + cb, len + cb, nullptr, status + j, ocap,
                                   reinterpret_cast<const double*>(st.t3 + size_t(hbase[k]) * sizeof(double)),
-                                  st.tile_base[k] * garena, lists + st.tile_base[k] * list_tile, s_lo + qb, s_hi + qb,
+                                  st.tile_base[k] * garena, lists + st.list_base[k], s_lo + qb, s_hi + qb,
                                   c_hi + cb, ax.sx, ax.sy};
         const int c = radius_class(rint);
         if (st.cls_t1[c] == 0) st.cls_t0[c] = st.tile_base[k];
