@@ -142,10 +142,11 @@ inline int direct_split(const Load& v, double R) {
 }
 // Whether the host has to know the endpoints (for the form, and small radii's splits).
 inline bool rules_count(double R) { return R < 6; }
+// Intervals a list has room for at first, and the most that later calls start with.
+constexpr int kListRoom = 24, kListRoomMost = 64;
 // Entries of a lane's interval list kept in LDS: the long list where columns
 // keep several intervals (small radii) or LDS does not decide how many waves
 // fit (split tiles), the short one elsewhere.
-constexpr int kListRoom = 24, kListRoomMost = 64;  // intervals a list starts with room for, and is kept at
 constexpr int kDirectListLong = 8, kDirectListShort = 3, kDirectSmallR = 3;
 inline int direct_list(int rint, int split) {
   return split > 1 || rint <= kDirectSmallR ? kDirectListLong : kDirectListShort;
@@ -293,6 +294,7 @@ struct vo_context {
   int dtab_axis = 0;
   int dtab_norder = 0;
   bool two_pass = false;  // VO_PASS1=zsweep, vo_pass1, vo_autotune: keep to the two sweeps
+  bool one_pass = false;  // VO_PASS1=direct: the one-pass form wherever it can, whatever is faster
   bool asked_sweeps = false;  // what the last device-held volume whose size was asked for took
   // intervals per list of the one-pass form, of single volumes and of batches
   // (whose memory it decides, see vo_list_capacity); each grows on overflow
@@ -1304,7 +1306,7 @@ DevVol dilate(vo_context* ctx, const DevVol& in, double R, int out_off_slot, int
   const auto fused = ctx->fused;
   bool by_rule = false;
   try {
-    return dilate_as<T>(ctx, in, R, out_off_slot, out_z_slot, t1, t2, &by_rule);
+    return dilate_as<T>(ctx, in, R, out_off_slot, out_z_slot, t1, t2, ctx->one_pass ? nullptr : &by_rule);
   } catch (const Failure& f) {
     if (f.code != VO_ERR_CAPACITY || !by_rule) throw;
   }
@@ -2735,6 +2737,7 @@ int vo_create(vo_context** out, int device) {
   if (const char* e = std::getenv("VO_PASS1")) {
     ctx->pass1_form = std::string(e) == "cull" ? 2 : (std::string(e) == "paint" ? 1 : 0);
     ctx->two_pass = std::string(e) == "zsweep";
+    ctx->one_pass = std::string(e) == "direct";
   }
   int rc = guarded(ctx, [&] {
     int n = 0;
